@@ -259,7 +259,8 @@ private:
 	DevLight* d_lights_ = nullptr;
 	float* d_gate_ = nullptr;     // shading factor per item (marched items)
 	uint32_t* d_mlist_ = nullptr; // compacted march list
-	uint32_t* d_mcount_ = nullptr; // [0] march count, [1] persistent-kernel cursor, [2] abort flag
+	uint32_t* d_mcount_ = nullptr; // [0] march count, then the march kernels' control words
+	void* d_long_ = nullptr;       // marches handed from a lane to a wave
 	uint32_t nmarch_ = 0;
 	unsigned persistent_blocks();
 	unsigned persist_blocks_ = 0;
