@@ -55,7 +55,7 @@ private:
 	void release();
 	void build_tiles();
 	void build_outliers();
-	void ensure_work();
+	void ensure_work(int form);
 	void ensure_part();
 	void ensure_perm_colors();
 	uint32_t ksplit(uint32_t rows_per_block, uint32_t min_blocks) const;
@@ -63,7 +63,7 @@ private:
 	// reduction prepares its operand (BF16) or its column scales (FP16)
 	void apply_dense(int form, const float* xT, float* yT, bool split, bool pre, bool chain = false);
 	void apply_tiles_f32(const float* xT, float* yT, bool pre);
-	void apply_op(int form, const double* x, double* y, bool pre);
+	void apply_op(int form, const double* x, double* y, bool pre, double* tot = nullptr);
 	DeviceScene& dev;
 	void* s_ = nullptr;
 	float* g32_ = nullptr;
@@ -94,9 +94,7 @@ private:
 	uint16_t* xqlo_ = nullptr;
 	float* xT_ = nullptr;
 	float* yT_ = nullptr;
-	float* rm32a_ = nullptr;
-	float* rm32b_ = nullptr;
-	float* rmx_ = nullptr;  // sparse FP32 forms: the operand (x diffuse) area prepared once per product
+	float* rmx_ = nullptr;  // sparse FP32 form: the operand (x diffuse) area prepared once per product
 	double* rmx64_ = nullptr; // the same for the FP64 form
 	unsigned* cmax_ = nullptr; // column maxima of the FP16 operand (its scales): two planes of kRPad
 	int cmax_cur_ = 0;         // the plane of the current operand

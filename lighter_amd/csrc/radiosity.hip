@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -992,63 +993,92 @@ __global__ __launch_bounds__(kB) void k_reduce_split(const float* __restrict__ p
 // ---------------------------------------------------------------------------
 // sparse gather over the symmetric CSR links.  The operand is prepared once
 // per product, xp[j][c] = (x[j][c] * diffuse[j][c % 3]) * area_j (PRE, the
-// reference's operation order) or x[j][c]; then one wave per row, lanes
-// over columns (up to 3 per lane for R <= 192), the row's links taken 64 at
-// a time (one coalesced load of columns and factors, broadcast lane by lane):
-// y[i][c] = sum_k xp[col_k][c] * f_k in link order.
+// reference's operation order) or x[j][c]; then one wave per row, the row's
+// links taken 64 at a time (one coalesced load of columns and factors):
+// y[i][c] = sum_k xp[col_k][c] * f_k, and tot[i][c] += y[i][c] (tot may be
+// null).
 // ---------------------------------------------------------------------------
 template <class T, bool PRE>
-__global__ __launch_bounds__(kB) void k_prep_rows(uint64_t n, uint32_t R, const T* __restrict__ x,
+__global__ __launch_bounds__(kB) void k_prep_rows(uint64_t n, uint32_t R, const double* __restrict__ x,
                                                   const float* __restrict__ diffuse, const float* __restrict__ area,
                                                   T* __restrict__ xp)
 {
 	const uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
 	if (t >= n)
 		return;
+	const T v = (T)x[t];
 	if (PRE) {
 		const uint32_t j = (uint32_t)(t / R), c = (uint32_t)(t % R);
-		xp[t] = (x[t] * (T)diffuse[3 * j + c % 3]) * (T)area[j];
+		xp[t] = (v * (T)diffuse[3 * j + c % 3]) * (T)area[j];
 	} else {
-		xp[t] = x[t];
+		xp[t] = v;
 	}
 }
 
-template <class T>
-__global__ __launch_bounds__(kB) void k_gather(uint32_t N, uint32_t R, const uint32_t* __restrict__ rowptr,
+// A lane holds column lane & (W - 1) (W the power of two at or above R, at
+// most 64; NJ = 3 columns, 64 apart, for wider operands) of the links
+// g, g + 64 / W, .. of each 64, g = lane / W; the groups' sums meet in a
+// butterfly.  So a row's 64 links are 64 operand rows in flight for one RGB
+// set-up (W = 4) instead of 64 loads of three lanes one after another, bound
+// by their latency (5,003 patches, 2.8 M entries, R = 3: 343 us a product;
+// a whole solve of 4 bounces 1,720 -> 237 us).  The order of the sum
+// is fixed; up to 64 columns it is 64 / W partial sums, wider it is the link
+// order.
+template <class T, int NJ>
+__global__ __launch_bounds__(kB) void k_gather(uint32_t N, uint32_t R, int logw, const uint32_t* __restrict__ rowptr,
                                                const uint32_t* __restrict__ col, const float* __restrict__ val,
-                                               const T* __restrict__ xp, T* __restrict__ y)
+                                               const T* __restrict__ xp, double* __restrict__ y,
+                                               double* __restrict__ tot)
 {
+	constexpr int U = 4; // link groups in flight
 	const uint32_t i = blockIdx.x * (kB / 64) + (threadIdx.x >> 6);
 	const int lane = threadIdx.x & 63;
 	if (i >= N)
 		return;
-	const uint32_t c0 = lane, c1 = lane + 64, c2 = lane + 128;
-	const bool u0 = c0 < R, u1 = c1 < R, u2 = c2 < R;
-	T a0 = 0, a1 = 0, a2 = 0;
+	const uint32_t c = (uint32_t)lane & ((1u << logw) - 1u), g = (uint32_t)lane >> logw, G = 64u >> logw;
+	T a[NJ];
+#pragma unroll
+	for (int j = 0; j < NJ; ++j)
+		a[j] = 0;
 	const uint32_t kb = rowptr[i], ke = rowptr[i + 1];
 	for (uint32_t k0 = kb; k0 < ke; k0 += 64) {
 		const uint32_t n = min(64u, ke - k0);
 		const uint32_t mj = (uint32_t)lane < n ? col[k0 + lane] : 0u;
 		const float mf = (uint32_t)lane < n ? val[k0 + lane] : 0.0f;
-		for (uint32_t q = 0; q < n; ++q) {
-			const uint32_t j = (uint32_t)__shfl((int)mj, (int)q);
-			const T f = (T)__shfl(mf, (int)q);
-			const T* row = xp + (uint64_t)j * R;
-			if (u0)
-				a0 += row[c0] * f;
-			if (u1)
-				a1 += row[c1] * f;
-			if (u2)
-				a2 += row[c2] * f;
+		for (uint32_t q = 0; q < n; q += U * G) {
+			T v[U][NJ], f[U];
+			bool in[U];
+#pragma unroll
+			for (int u = 0; u < U; ++u) {
+				const uint32_t k = q + u * G + g;
+				in[u] = k < n;
+				const uint32_t jj = (uint32_t)__shfl((int)mj, (int)(k & 63u));
+				f[u] = (T)__shfl(mf, (int)(k & 63u));
+#pragma unroll
+				for (int j = 0; j < NJ; ++j)
+					v[u][j] = in[u] && c + 64 * j < R ? xp[(uint64_t)jj * R + c + 64 * j] : (T)0;
+			}
+#pragma unroll
+			for (int u = 0; u < U; ++u)
+#pragma unroll
+				for (int j = 0; j < NJ; ++j)
+					if (in[u])
+						a[j] += v[u][j] * f[u];
 		}
 	}
-	T* out = y + (uint64_t)i * R;
-	if (u0)
-		out[c0] = a0;
-	if (u1)
-		out[c1] = a1;
-	if (u2)
-		out[c2] = a2;
+	for (int o = 1 << logw; o < 64; o <<= 1)
+#pragma unroll
+		for (int j = 0; j < NJ; ++j)
+			a[j] += __shfl_xor(a[j], o);
+	if (g == 0)
+#pragma unroll
+		for (int j = 0; j < NJ; ++j)
+			if (c + 64 * j < R) {
+				const uint64_t o = (uint64_t)i * R + c + 64 * j;
+				y[o] = (double)a[j];
+				if (tot)
+					tot[o] += (double)a[j];
+			}
 }
 
 // layout changes between the row-major (sparse) and column-major (dense) sets
@@ -1074,13 +1104,6 @@ __global__ void k_to_rowmajor(const A* __restrict__ xT, uint32_t N, uint32_t Np,
 		return;
 	uint32_t j = (uint32_t)(t / R), c = (uint32_t)(t % R);
 	x[t] = (B)xT[(uint64_t)c * Np + (pinv ? pinv[j] : j)];
-}
-
-template <class A, class B> __global__ void k_copy_cast(uint64_t n, const A* __restrict__ x, B* __restrict__ y)
-{
-	uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
-	if (t < n)
-		y[t] = (B)x[t];
 }
 
 template <class A, class B> __global__ void k_axpy(uint64_t n, const A* __restrict__ x, B* __restrict__ y)
@@ -1185,8 +1208,6 @@ void RadSolver::release()
 	dfree(xqlo_);
 	dfree(xT_);
 	dfree(yT_);
-	dfree(rm32a_);
-	dfree(rm32b_);
 	dfree(rmx_);
 	dfree(rmx64_);
 	dfree(cmax_);
@@ -1203,8 +1224,6 @@ void RadSolver::set_problem(const double* E, uint32_t R_, const float* diffuse3,
 	if (R_ == 0 || R_ > (uint32_t)kRPad)
 		throw std::runtime_error("RadSolver: 1..192 right-hand sides");
 	if (R_ != R) {
-		dfree(rm32a_);
-		dfree(rm32b_);
 		dfree(rmx_);
 		dfree(rmx64_);
 	}
@@ -1480,23 +1499,22 @@ void RadSolver::ensure_part()
 }
 
 // work buffers of the products (kept across solves)
-void RadSolver::ensure_work()
+void RadSolver::ensure_work(int form)
 {
 	const uint64_t n = (uint64_t)kRPad * Np;
-	ensure_part();
-	if (!xq_) {
+	if (form >= kDenseF32)
+		ensure_part();
+	if (form >= kDenseF32 && !xq_) {
 		xq_ = dalloc<float>(n); // FP32 operand, or the 16-bit one in its first half
 		xqlo_ = dalloc<uint16_t>(n);
 		xT_ = dalloc<float>(n);
 		yT_ = dalloc<float>(n);
 		cmax_ = dalloc<unsigned>(2 * kRPad);
 	}
-	if (!rm32a_) {
-		rm32a_ = dalloc<float>((uint64_t)Np * R);
-		rm32b_ = dalloc<float>((uint64_t)Np * R);
+	if (form == kSparseF32 && !rmx_)
 		rmx_ = dalloc<float>((uint64_t)Np * R);
+	if (form == kSparseF64 && !rmx64_)
 		rmx64_ = dalloc<double>((uint64_t)Np * R);
-	}
 }
 
 // y = K x (pre) or H x over the FP32 tile store (Morton order in and out)
@@ -1636,8 +1654,9 @@ void RadSolver::apply_dense(int form, const float* xT, float* yT, bool split, bo
 	HIPCHECK(hipGetLastError());
 }
 
-// y = K x (pre) or H x, row-major N x R FP64 in and out, in the given form
-void RadSolver::apply_op(int form, const double* x, double* y, bool pre)
+// y = K x (pre) or H x, row-major N x R FP64 in and out, in the given form;
+// tot += y when tot is given
+void RadSolver::apply_op(int form, const double* x, double* y, bool pre, double* tot)
 {
 	hipStream_t s = (hipStream_t)s_;
 	const uint64_t nR = (uint64_t)N * R, nRp = (uint64_t)R * Np;
@@ -1645,25 +1664,32 @@ void RadSolver::apply_op(int form, const double* x, double* y, bool pre)
 	const uint32_t* rp = dev.rad.rowptr;
 	const uint32_t* cl = dev.rad.col;
 	const float* vl = dev.rad.val;
-	if (form == kSparseF64) {
-		if (pre)
-			k_prep_rows<double, true><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, rmx64_);
+	if (form == kSparseF64 || form == kSparseF32) {
+		auto product = [&](auto* xp) {
+			using T = std::remove_pointer_t<decltype(xp)>;
+			if (pre)
+				k_prep_rows<T, true><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, xp);
+			else
+				k_prep_rows<T, false><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, xp);
+			int logw = 0;
+			while (logw < 6 && (1u << logw) < R)
+				++logw;
+			if (R <= 64)
+				k_gather<T, 1><<<sgrid, kB, 0, s>>>(N, R, logw, rp, cl, vl, xp, y, tot);
+			else
+				k_gather<T, 3><<<sgrid, kB, 0, s>>>(N, R, logw, rp, cl, vl, xp, y, tot);
+		};
+		if (form == kSparseF64)
+			product(rmx64_);
 		else
-			k_prep_rows<double, false><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, rmx64_);
-		k_gather<double><<<sgrid, kB, 0, s>>>(N, R, rp, cl, vl, rmx64_, y);
-	} else if (form == kSparseF32) {
-		k_copy_cast<double, float><<<gridn(nR), kB, 0, s>>>(nR, x, rm32a_);
-		if (pre)
-			k_prep_rows<float, true><<<gridn(nR), kB, 0, s>>>(nR, R, rm32a_, diff_, area_, rmx_);
-		else
-			k_prep_rows<float, false><<<gridn(nR), kB, 0, s>>>(nR, R, rm32a_, diff_, area_, rmx_);
-		k_gather<float><<<sgrid, kB, 0, s>>>(N, R, rp, cl, vl, rmx_, rm32b_);
-		k_copy_cast<float, double><<<gridn(nR), kB, 0, s>>>(nR, rm32b_, y);
+			product(rmx_);
 	} else {
 		const bool mo = storage_of(form) != kDenseF32; // Morton order
 		k_to_colmajor<double, float><<<gridn(nRp), kB, 0, s>>>(x, N, Np, R, mo ? perm_ : nullptr, xT_);
 		apply_dense(form, xT_, yT_, false, pre);
 		k_to_rowmajor<float, double><<<gridn(nR), kB, 0, s>>>(yT_, N, Np, R, mo ? pinv_ : nullptr, y);
+		if (tot)
+			k_axpy<double, double><<<gridn(nR), kB, 0, s>>>(nR, y, tot);
 	}
 	HIPCHECK(hipGetLastError());
 }
@@ -1678,7 +1704,7 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 	hipStream_t s = (hipStream_t)s_;
 	uint64_t nR = (uint64_t)N * R, nRp = (uint64_t)R * Np;
 	times = RadTimes{};
-	ensure_work();
+	ensure_work(form);
 	// FP64 running total
 	DevBuf<double> tot(nR);
 	HIPCHECK(hipMemcpyAsync(tot, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
@@ -1687,8 +1713,7 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 		HIPCHECK(hipMemcpyAsync(x, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
 		Ev ev(s);
 		for (int b = 0; b < bounces; ++b) {
-			apply_op(form, x, y, true);
-			k_axpy<double, double><<<gridn(nR), kB, 0, s>>>(nR, y, tot);
+			apply_op(form, x, y, true, tot);
 			std::swap(x, y);
 		}
 		times.series_ms = ev.stop();
@@ -1768,7 +1793,7 @@ void RadSolver::solve_grad(int form, int bounces, const double* g, double* total
 	hipStream_t s = (hipStream_t)s_;
 	const uint64_t nR = (uint64_t)N * R;
 	times = RadTimes{};
-	ensure_work();
+	ensure_work(form);
 	if (form >= kDenseF32 && built_form_ != storage_of(form))
 		build_dense(form);
 	const int B = std::max(0, bounces);
@@ -1782,8 +1807,7 @@ void RadSolver::solve_grad(int form, int bounces, const double* g, double* total
 	HIPCHECK(hipMemcpyAsync(z, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
 	HIPCHECK(hipMemcpyAsync(tot, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
 	for (int k = 1; k <= B; ++k) {
-		apply_op(form, z, zn, true);
-		k_axpy<double, double><<<gridn(nR), kB, 0, s>>>(nR, zn, tot);
+		apply_op(form, z, zn, true, tot);
 		if (k < B)
 			HIPCHECK(hipMemcpyAsync(S[k], tot, 8 * nR, hipMemcpyDeviceToDevice, s));
 		std::swap(z, zn);
