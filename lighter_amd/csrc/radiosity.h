@@ -107,6 +107,7 @@ private:
 	// by the reduction (CSR by Morton position), the rest go to the tiles
 	uint32_t* orow_ = nullptr;
 	uint32_t* ocol_ = nullptr;
+	uint32_t* opos_ = nullptr;
 	float* oval_ = nullptr;
 	uint64_t nout_ = 0;
 	float othr_ = 0.0f;

@@ -256,7 +256,7 @@ __global__ __launch_bounds__(kB) void k_outlier_fill(uint32_t N, const uint32_t*
                                                      const uint32_t* __restrict__ col, const float* __restrict__ val,
                                                      float thr, const uint32_t* __restrict__ pinv,
                                                      const uint32_t* __restrict__ orow, uint32_t* __restrict__ ocol,
-                                                     float* __restrict__ oval)
+                                                     uint32_t* __restrict__ opos, float* __restrict__ oval)
 {
 	const uint32_t i = blockIdx.x * (kB / 64) + (threadIdx.x >> 6);
 	const int lane = threadIdx.x & 63;
@@ -270,6 +270,7 @@ __global__ __launch_bounds__(kB) void k_outlier_fill(uint32_t N, const uint32_t*
 		if (hit) {
 			const uint32_t at = o + (uint32_t)__popcll(m & ((1ull << lane) - 1));
 			ocol[at] = pinv[col[k]];
+			opos[at] = pinv[i];
 			oval[at] = val[k];
 		}
 		o += (uint32_t)__popcll(m);
@@ -349,15 +350,17 @@ struct OperandPass {
 	// the product's FP32 operand w_in (from its input vector xin)
 	const uint32_t* orow = nullptr;
 	const uint32_t* ocol = nullptr;
+	const uint32_t* opos = nullptr; // each outlier's own position
 	const float* oval = nullptr;
 	const float* xin = nullptr;
 	uint32_t Np = 0, R = 0;
+	uint32_t ncg = kRPad / 16; // column groups with live columns
 };
 
 template <int P>
 __global__ __launch_bounds__(kB) void k_operand(const OperandPass a)
 {
-	const uint32_t cg = blockIdx.x % (kRPad / 16), rb = blockIdx.x / (kRPad / 16);
+	const uint32_t cg = blockIdx.x % a.ncg, rb = blockIdx.x / a.ncg;
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane >> 2, pc = lane & 3;
 	const uint32_t c = cg * 16 + r;
 	const bool live = c < a.R;
@@ -370,6 +373,72 @@ __global__ __launch_bounds__(kB) void k_operand(const OperandPass a)
 	}
 	const float sc = a.xq ? col_scale_of(a.cmax_op, c) : 1.0f;
 	float m = 0.0f;
+	// The row block's outliers first: its entries (in row order) in 16 equal
+	// runs, a thread per (run, column).  A run adds up its rows one after
+	// another, four entries in flight; what it holds of a row that began in
+	// an earlier run is added afterwards, in run order, so the sums do not
+	// depend on timing.  Near an edge of two surfaces a few rows hold most of
+	// the entries: on 32,768 patches of a room with 192 columns a pass took
+	// 198 us with a lane summing its own eight rows, 125 us with a thread per
+	// row and 98 us so.
+	__shared__ float out[16][257], head[16][17];
+	__shared__ uint32_t head_row[16];
+	const uint32_t o0 = a.part && a.orow ? a.orow[rb * 256] : 0, o1 = a.part && a.orow ? a.orow[rb * 256 + 256] : 0;
+	const bool outliers = o0 != o1;
+	if (outliers) {
+		const uint32_t oc = threadIdx.x & 15, run = threadIdx.x >> 4, col = cg * 16 + oc;
+		for (uint32_t p = run; p < 256; p += 16)
+			out[oc][p] = 0.0f;
+		__syncthreads();
+		const uint32_t k0 = o0 + (uint32_t)((uint64_t)(o1 - o0) * run / 16);
+		const uint32_t k1 = o0 + (uint32_t)((uint64_t)(o1 - o0) * (run + 1) / 16);
+		const float* xin = a.xin + (uint64_t)(col < a.R ? col : 0) * a.Np;
+		uint32_t row = k0 < k1 ? a.opos[k0] & 255u : 0u;
+		bool begun = k0 < k1 && a.orow[rb * 256 + row] < k0; // by an earlier run
+		float sum = 0.0f, first = 0.0f;
+		if (oc == 0)
+			head_row[run] = row;
+		for (uint32_t k = k0; k < k1; k += 4) {
+			float w[4];
+			uint32_t r4[4];
+#pragma unroll
+			for (int u = 0; u < 4; ++u) {
+				const uint32_t kk = min(k + u, k1 - 1), q = a.ocol[kk];
+				r4[u] = a.opos[kk] & 255u;
+				w[u] = xin[q];
+				if (a.pre)
+					w[u] = (w[u] * a.dperm[3 * q + col % 3]) * a.aperm[q];
+				w[u] *= a.oval[kk];
+			}
+#pragma unroll
+			for (int u = 0; u < 4; ++u) {
+				if (k + u >= k1)
+					break;
+				if (r4[u] != row) {
+					if (begun)
+						first = sum;
+					else
+						out[oc][row] = sum;
+					begun = false;
+					row = r4[u];
+					sum = 0.0f;
+				}
+				sum += w[u];
+			}
+		}
+		if (k0 < k1) {
+			if (begun)
+				first = sum;
+			else
+				out[oc][row] = sum;
+		}
+		head[run][oc] = first;
+		__syncthreads();
+		if (threadIdx.x < 16)
+			for (int g = 0; g < 16; ++g)
+				out[oc][head_row[g]] += head[g][oc];
+		__syncthreads();
+	}
 #pragma unroll
 	for (int k = 0; k < 2; ++k) {
 		const uint32_t stage = rb * 8 + wave * 2 + k, j0 = stage * 32 + pc * 8;
@@ -388,16 +457,10 @@ __global__ __launch_bounds__(kB) void k_operand(const OperandPass a)
 #pragma unroll
 			for (int e = 0; e < 8; ++e)
 				v[e] *= inv;
-			if (a.orow && live && a.orow[j0] != a.orow[j0 + 8]) {
+			if (outliers)
+#pragma unroll
 				for (int e = 0; e < 8; ++e)
-					for (uint32_t k = a.orow[j0 + e]; k < a.orow[j0 + e + 1]; ++k) {
-						const uint32_t q = a.ocol[k];
-						float w = a.xin[cbase + q];
-						if (a.pre)
-							w = (w * a.dperm[3 * q + c % 3]) * a.aperm[q];
-						v[e] += a.oval[k] * w;
-					}
-			}
+					v[e] += out[r][(wave * 2 + k) * 32 + pc * 8 + e];
 		} else if (live) {
 			const float4 u0 = *reinterpret_cast<const float4*>(a.x + cbase + j0);
 			const float4 u1 = *reinterpret_cast<const float4*>(a.x + cbase + j0 + 4);
@@ -549,10 +612,10 @@ __device__ __forceinline__ void dma16(const uint16_t* src, unsigned char* dst)
 // product, so its loads are non-temporal: they leave the L2 to the operand
 // stages, which every row block of the same k stage reads again.
 // ---------------------------------------------------------------------------
-template <int NPL, int D>
+template <int NPL, int D, int NC>
 struct TileLane {
-	static constexpr int kXPlane = kRPad * kKS * 2; // operand plane per stage (12 KB)
-	static constexpr int kOps = NPL * (3 + 4);      // loads and copies per wave per stage
+	static constexpr int kXPlane = NC * 16 * kKS * 2; // operand plane per stage (12 KB for 12 column tiles)
+	static constexpr int kOps = NPL * (NC / 4 + 4);   // loads and copies per wave per stage
 	const uint16_t *G, *Glo, *xq, *xlo;
 	const uint32_t* lst; // k stages of the run's tiles
 	uint64_t first;      // the run's first tile
@@ -569,22 +632,22 @@ __device__ __forceinline__ void lds_reads_done()
 	asm volatile("" ::: "memory");
 }
 
-template <int NPL, int D>
-__device__ __forceinline__ void tile_copy_operand(const TileLane<NPL, D>& L, uint32_t st, unsigned char* slot)
+template <int NPL, int D, int NC>
+__device__ __forceinline__ void tile_copy_operand(const TileLane<NPL, D, NC>& L, uint32_t st, unsigned char* slot)
 {
 	const uint64_t ks = L.lst[st];
 #pragma unroll
 	for (int pl = 0; pl < NPL; ++pl) {
 		const uint16_t* X = (pl ? L.xlo : L.xq) + ks * kXStageElems + 8 * L.lane;
 #pragma unroll
-		for (int j = 0; j < 3; ++j)
-			dma16(X + (uint64_t)(3 * L.wave + j) * kTileElems,
-			      slot + pl * TileLane<NPL, D>::kXPlane + (3 * L.wave + j) * 1024);
+		for (int j = 0; j < NC / 4; ++j)
+			dma16(X + (uint64_t)(NC / 4 * L.wave + j) * kTileElems,
+			      slot + pl * TileLane<NPL, D, NC>::kXPlane + (NC / 4 * L.wave + j) * 1024);
 	}
 }
 
-template <int NPL, int D>
-__device__ __forceinline__ void tile_load_matrix(const TileLane<NPL, D>& L, uint32_t st, i16x8 (&a)[NPL][4])
+template <int NPL, int D, int NC>
+__device__ __forceinline__ void tile_load_matrix(const TileLane<NPL, D, NC>& L, uint32_t st, i16x8 (&a)[NPL][4])
 {
 	const uint64_t base = (L.first + st) * kGStageElems + (uint64_t)(4 * L.wave) * kTileElems + L.aofs;
 #pragma unroll
@@ -596,26 +659,26 @@ __device__ __forceinline__ void tile_load_matrix(const TileLane<NPL, D>& L, uint
 	}
 }
 
-template <int P, int NPL, int D, int B>
-__device__ __forceinline__ void tile_step(int s, int nst, const TileLane<NPL, D>& L, i16x8 (&a)[D][NPL][4],
-                                          f32x4 (&acc)[4][kColTiles])
+template <int P, int NPL, int D, int NC, int B>
+__device__ __forceinline__ void tile_step(int s, int nst, const TileLane<NPL, D, NC>& L, i16x8 (&a)[D][NPL][4],
+                                          f32x4 (&acc)[4][NC])
 {
-	typedef TileLane<NPL, D> T;
+	typedef TileLane<NPL, D, NC> T;
 	wait_vm<T::kOps * (D - 1)>();
 	block_barrier();
 	unsigned char* slot = L.slot[B];
-	i16x8 bx[NPL][kColTiles];
+	i16x8 bx[NPL][NC];
 #pragma unroll
 	for (int pl = 0; pl < NPL; ++pl)
 #pragma unroll
-		for (int c = 0; c < kColTiles; ++c)
+		for (int c = 0; c < NC; ++c)
 			bx[pl][c] = *reinterpret_cast<const i16x8*>(slot + pl * T::kXPlane + c * 1024 + L.rofs);
 	lds_reads_done();
 	block_barrier();
 	const int ahead = s + D < nst ? s + D : nst - 1;
-	tile_copy_operand<NPL, D>(L, (uint32_t)ahead, slot);
+	tile_copy_operand<NPL, D, NC>(L, (uint32_t)ahead, slot);
 #pragma unroll
-	for (int c = 0; c < kColTiles; ++c) {
+	for (int c = 0; c < NC; ++c) {
 #pragma unroll
 		for (int t = 0; t < 4; ++t)
 			acc[t][c] = mfma16<P>(a[B][0][t], bx[0][c], acc[t][c]);
@@ -628,33 +691,33 @@ __device__ __forceinline__ void tile_step(int s, int nst, const TileLane<NPL, D>
 			}
 		}
 	}
-	tile_load_matrix<NPL, D>(L, (uint32_t)ahead, a[B]);
+	tile_load_matrix<NPL, D, NC>(L, (uint32_t)ahead, a[B]);
 }
 
-template <int P, int NPL, int D, int... Bs>
-__device__ __forceinline__ void tile_steps(int s, int nst, const TileLane<NPL, D>& L, i16x8 (&a)[D][NPL][4],
-                                           f32x4 (&acc)[4][kColTiles], std::integer_sequence<int, Bs...>)
+template <int P, int NPL, int D, int NC, int... Bs>
+__device__ __forceinline__ void tile_steps(int s, int nst, const TileLane<NPL, D, NC>& L, i16x8 (&a)[D][NPL][4],
+                                           f32x4 (&acc)[4][NC], std::integer_sequence<int, Bs...>)
 {
-	(tile_step<P, NPL, D, Bs>(s + Bs, nst, L, a, acc), ...);
+	(tile_step<P, NPL, D, NC, Bs>(s + Bs, nst, L, a, acc), ...);
 }
 
-template <int P, int NPL, int D, int... Bs>
-__device__ __forceinline__ void tile_tail(int s, int nst, const TileLane<NPL, D>& L, i16x8 (&a)[D][NPL][4],
-                                          f32x4 (&acc)[4][kColTiles], std::integer_sequence<int, Bs...>)
+template <int P, int NPL, int D, int NC, int... Bs>
+__device__ __forceinline__ void tile_tail(int s, int nst, const TileLane<NPL, D, NC>& L, i16x8 (&a)[D][NPL][4],
+                                          f32x4 (&acc)[4][NC], std::integer_sequence<int, Bs...>)
 {
-	((s + Bs < nst ? tile_step<P, NPL, D, Bs>(s + Bs, nst, L, a, acc) : void()), ...);
+	((s + Bs < nst ? tile_step<P, NPL, D, NC, Bs>(s + Bs, nst, L, a, acc) : void()), ...);
 }
 
-template <int NPL, int D, int... Bs>
-__device__ __forceinline__ void tile_prologue(int nst, const TileLane<NPL, D>& L, i16x8 (&a)[D][NPL][4],
+template <int NPL, int D, int NC, int... Bs>
+__device__ __forceinline__ void tile_prologue(int nst, const TileLane<NPL, D, NC>& L, i16x8 (&a)[D][NPL][4],
                                               std::integer_sequence<int, Bs...>)
 {
-	((tile_copy_operand<NPL, D>(L, (uint32_t)(Bs < nst ? Bs : nst - 1), L.slot[Bs]),
-	  tile_load_matrix<NPL, D>(L, (uint32_t)(Bs < nst ? Bs : nst - 1), a[Bs])),
+	((tile_copy_operand<NPL, D, NC>(L, (uint32_t)(Bs < nst ? Bs : nst - 1), L.slot[Bs]),
+	  tile_load_matrix<NPL, D, NC>(L, (uint32_t)(Bs < nst ? Bs : nst - 1), a[Bs])),
 	 ...);
 }
 
-template <int P, int NPL, int D>
+template <int P, int NPL, int D, int NC>
 __global__ __launch_bounds__(kB) void k_gemm_tiles(const uint16_t* __restrict__ G, const uint16_t* __restrict__ Glo,
                                                    const uint16_t* __restrict__ xq, const uint16_t* __restrict__ xlo,
                                                    const uint4* __restrict__ chunks,
@@ -662,8 +725,9 @@ __global__ __launch_bounds__(kB) void k_gemm_tiles(const uint16_t* __restrict__ 
                                                    const uint32_t* __restrict__ tks, uint32_t Np,
                                                    float* __restrict__ part)
 {
-	typedef TileLane<NPL, D> T;
+	typedef TileLane<NPL, D, NC> T;
 	static_assert(D >= 2 && D <= kMaxPD, "ring depth");
+	static_assert(NC % 4 == 0 && NC <= kColTiles, "each wave copies NC / 4 of a stage's column groups");
 	constexpr int kSlot = NPL * T::kXPlane;
 	__shared__ __align__(1024) unsigned char lds0[kSlot], lds1[kSlot], lds2[D > 2 ? kSlot : 16],
 	    lds3[D > 3 ? kSlot : 16], lds4[D > 4 ? kSlot : 16], lds5[D > 5 ? kSlot : 16];
@@ -693,19 +757,19 @@ __global__ __launch_bounds__(kB) void k_gemm_tiles(const uint16_t* __restrict__ 
 		const int nst = (int)(ch.z - ch.y);
 		L.lst = tks + ch.y;
 		L.first = ch.y;
-		f32x4 acc[4][kColTiles];
+		f32x4 acc[4][NC];
 #pragma unroll
 		for (int t = 0; t < 4; ++t)
 #pragma unroll
-			for (int c = 0; c < kColTiles; ++c)
+			for (int c = 0; c < NC; ++c)
 				acc[t][c] = f32x4{0, 0, 0, 0};
 		if (nst > 0) {
 			i16x8 a[D][NPL][4];
-			tile_prologue<NPL, D>(nst, L, a, std::make_integer_sequence<int, D>{});
+			tile_prologue<NPL, D, NC>(nst, L, a, std::make_integer_sequence<int, D>{});
 			int s = 0;
 			for (; s + D <= nst; s += D)
-				tile_steps<P, NPL, D>(s, nst, L, a, acc, std::make_integer_sequence<int, D>{});
-			tile_tail<P, NPL, D>(s, nst, L, a, acc, std::make_integer_sequence<int, D - 1>{});
+				tile_steps<P, NPL, D, NC>(s, nst, L, a, acc, std::make_integer_sequence<int, D>{});
+			tile_tail<P, NPL, D, NC>(s, nst, L, a, acc, std::make_integer_sequence<int, D - 1>{});
 			wait_vm<0>();    // no copy lands after the segment (or the block) is done with the ring
 			block_barrier(); // every wave has finished with the ring before the next segment refills it
 		}
@@ -713,7 +777,7 @@ __global__ __launch_bounds__(kB) void k_gemm_tiles(const uint16_t* __restrict__ 
 #pragma unroll
 		for (int t = 0; t < 4; ++t)
 #pragma unroll
-			for (int c = 0; c < kColTiles; ++c) {
+			for (int c = 0; c < NC; ++c) {
 				const uint32_t col = c * 16 + r, i = i0 + t * 16 + 4 * g;
 				*reinterpret_cast<float4*>(out + (uint64_t)col * Np + i) =
 				    make_float4(acc[t][c][0], acc[t][c][1], acc[t][c][2], acc[t][c][3]);
@@ -721,7 +785,14 @@ __global__ __launch_bounds__(kB) void k_gemm_tiles(const uint16_t* __restrict__ 
 	}
 }
 
-constexpr int kTilesD1 = 4, kTilesD2 = 3; // ring depths of the plain and compensated products
+// Ring depths of the plain and compensated products, and the column tiles
+// they take (a multiple of four: 16-column tiles 4, 8 or 12).  With few
+// right-hand sides the matrix stream is all there is, so fewer columns mean
+// deeper rings of smaller stages, a third of the operand copies and of the
+// partial sums (24,001 patches of a room, R = 3: 184 -> 138 us a product, of
+// 770 MB of matrix).
+constexpr int ring_depth(int npl, int nc) { return nc == 4 ? (npl == 1 ? 6 : 4) : (npl == 1 ? 4 : 3); }
+static inline int col_tiles(uint32_t R) { return R <= 64 ? 4 : R <= 128 ? 8 : 12; }
 
 constexpr uint32_t kMaxSlots = 16; // partial-sum planes allocated at least
 constexpr uint64_t kMinShare = 16;  // fewest tiles per persistent block of the tile products
@@ -748,8 +819,7 @@ constexpr uint64_t kMinShare = 16;  // fewest tiles per persistent block of the 
 constexpr uint64_t kT32Group = 512;                      // floats per 2 KB group
 constexpr uint64_t kT32Tile = 16 * kT32Group;            // a stored tile
 constexpr uint64_t kT32XStage = (kRPad / 16) * kT32Group; // an operand stage
-constexpr int kT32XBytes = (int)(kT32XStage * 4);          // 24 KB
-constexpr int kT32Stage = kT32XBytes + (int)(kT32Tile * 4); // 56 KB
+constexpr int t32_stage(int nc) { return nc * 2048 + (int)(kT32Tile * 4); } // 56 KB for 12 column tiles
 
 __device__ __forceinline__ int t32_slot(int piece, int row) { return piece ^ (row & 7); }
 
@@ -759,6 +829,7 @@ __device__ __forceinline__ void dma16f(const float* src, unsigned char* dst)
 }
 
 // stage st of the run (tile first + st, operand stage lst[st]) into buf
+template <int NC>
 __device__ __forceinline__ void t32_issue(const float* G, const float* xq, uint64_t first, const uint32_t* lst,
                                           uint32_t st, unsigned char* buf, int wave, int lane)
 {
@@ -766,13 +837,14 @@ __device__ __forceinline__ void t32_issue(const float* G, const float* xq, uint6
 	const float* xs = xq + ks * kT32XStage + 4 * lane;
 	const float* gs = G + (first + st) * kT32Tile + 4 * lane;
 #pragma unroll
-	for (int j = 0; j < 6; ++j) // the operand's 24 KB: 6 per wave
-		dma16f(xs + (uint64_t)(6 * wave + j) * 256, buf + (6 * wave + j) * 1024);
+	for (int j = 0; j < NC / 2; ++j) // the operand's 2 KB a column tile (24 KB for 12): NC / 2 copies per wave
+		dma16f(xs + (uint64_t)(NC / 2 * wave + j) * 256, buf + (NC / 2 * wave + j) * 1024);
 #pragma unroll
 	for (int j = 0; j < 8; ++j) // the wave's own 64 rows: 4 groups of 2 KB
-		dma16f(gs + (uint64_t)(8 * wave + j) * 256, buf + kT32XBytes + (8 * wave + j) * 1024);
+		dma16f(gs + (uint64_t)(8 * wave + j) * 256, buf + NC * 2048 + (8 * wave + j) * 1024);
 }
 
+template <int NC>
 __global__ __launch_bounds__(kB) void k_gemm_f32t(const float* __restrict__ G, const float* __restrict__ xq,
                                                   const uint4* __restrict__ chunks,
                                                   const uint32_t* __restrict__ seg_off,
@@ -780,7 +852,7 @@ __global__ __launch_bounds__(kB) void k_gemm_f32t(const float* __restrict__ G, c
                                                   float* __restrict__ part)
 {
 	constexpr int RT = 4; // row tiles per wave
-	__shared__ __align__(1024) unsigned char lds0[kT32Stage], lds1[kT32Stage];
+	__shared__ __align__(1024) unsigned char lds0[t32_stage(NC)], lds1[t32_stage(NC)];
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int r = lane & 15, g = lane >> 4;
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -794,42 +866,42 @@ __global__ __launch_bounds__(kB) void k_gemm_f32t(const float* __restrict__ G, c
 	const int nst = (int)(ch.z - ch.y);
 	const uint32_t* lst = tks + ch.y;
 
-	f32x4 acc[RT][kColTiles];
+	f32x4 acc[RT][NC];
 #pragma unroll
 	for (int t = 0; t < RT; ++t)
 #pragma unroll
-		for (int c = 0; c < kColTiles; ++c)
+		for (int c = 0; c < NC; ++c)
 			acc[t][c] = f32x4{0, 0, 0, 0};
 
 	for (int st = 0; st < nst; ++st) {
 		unsigned char* cur = (st & 1) ? lds1 : lds0;
 		unsigned char* nxt = (st & 1) ? lds0 : lds1;
 		if (st == 0)
-			t32_issue(G, xq, ch.y, lst, 0, cur, wave, lane);
+			t32_issue<NC>(G, xq, ch.y, lst, 0, cur, wave, lane);
 		wait_vm<0>();    // this wave's part of stage st has landed
 		block_barrier(); // every wave's part is in; stage st-1's buffer is free
-		float4 a[RT][2], b[kColTiles][2];
+		float4 a[RT][2], b[NC][2];
 #pragma unroll
 		for (int t = 0; t < RT; ++t) {
-			const unsigned char* rowp = cur + kT32XBytes + (wave * RT + t) * 2048 + r * 128;
+			const unsigned char* rowp = cur + NC * 2048 + (wave * RT + t) * 2048 + r * 128;
 			a[t][0] = *reinterpret_cast<const float4*>(rowp + s0);
 			a[t][1] = *reinterpret_cast<const float4*>(rowp + s1);
 		}
 #pragma unroll
-		for (int c = 0; c < kColTiles; ++c) {
+		for (int c = 0; c < NC; ++c) {
 			const unsigned char* colp = cur + c * 2048 + r * 128;
 			b[c][0] = *reinterpret_cast<const float4*>(colp + s0);
 			b[c][1] = *reinterpret_cast<const float4*>(colp + s1);
 		}
 		// every fragment is read before the next DMA is issued (see gemm_step)
 		if (st + 1 < nst)
-			t32_issue(G, xq, ch.y, lst, st + 1, nxt, wave, lane);
+			t32_issue<NC>(G, xq, ch.y, lst, st + 1, nxt, wave, lane);
 #pragma unroll
 		for (int e = 0; e < 8; ++e)
 #pragma unroll
 			for (int t = 0; t < RT; ++t)
 #pragma unroll
-				for (int c = 0; c < kColTiles; ++c) {
+				for (int c = 0; c < NC; ++c) {
 					const float av = e < 4 ? a[t][0][e] : a[t][1][e - 4];
 					const float bv = e < 4 ? b[c][0][e] : b[c][1][e - 4];
 					acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[t][c], 0, 0, 0);
@@ -840,7 +912,7 @@ __global__ __launch_bounds__(kB) void k_gemm_f32t(const float* __restrict__ G, c
 #pragma unroll
 	for (int t = 0; t < RT; ++t)
 #pragma unroll
-		for (int c = 0; c < kColTiles; ++c) {
+		for (int c = 0; c < NC; ++c) {
 			const uint32_t col = c * 16 + r, i = i0 + t * 16 + 4 * g;
 			*reinterpret_cast<float4*>(out + (uint64_t)col * Np + i) =
 			    make_float4(acc[t][c][0], acc[t][c][1], acc[t][c][2], acc[t][c][3]);
@@ -877,12 +949,12 @@ __global__ __launch_bounds__(kB) void k_tile_scatter_f32(uint32_t N, uint32_t Np
 // x[c][j], in the LDS-image layout: stage j / 32, column group c / 16, row
 // c % 16, piece (j % 32) / 4 at slot piece ^ (c % 8)
 __global__ __launch_bounds__(kB) void k_prep_x32t(const float* __restrict__ xT, const float* __restrict__ dperm,
-                                                  const float* __restrict__ aperm, uint32_t Np, uint32_t R, int pre,
-                                                  float* __restrict__ xq)
+                                                  const float* __restrict__ aperm, uint32_t Np, uint32_t R,
+                                                  uint32_t cols, int pre, float* __restrict__ xq)
 {
 	const uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
 	const uint32_t pieces = Np / 4;
-	if (t >= (uint64_t)kRPad * pieces)
+	if (t >= (uint64_t)cols * pieces)
 		return;
 	const uint32_t c = (uint32_t)(t / pieces), j0 = (uint32_t)(t % pieces) * 4;
 	float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1215,6 +1287,7 @@ void RadSolver::release()
 	dfree(aperm_);
 	dfree(orow_);
 	dfree(ocol_);
+	dfree(opos_);
 	dfree(oval_);
 }
 
@@ -1409,6 +1482,7 @@ void RadSolver::build_outliers()
 	nout_ = cum;
 	dfree(orow_);
 	dfree(ocol_);
+	dfree(opos_);
 	dfree(oval_);
 	if (nout_) {
 		DevBuf<uint32_t> cnt(Np);
@@ -1423,10 +1497,11 @@ void RadSolver::build_outliers()
 			throw std::runtime_error("RadSolver: outlier count differs from the histogram");
 		orow_ = dalloc<uint32_t>(Np + 1);
 		ocol_ = dalloc<uint32_t>(nout_);
+		opos_ = dalloc<uint32_t>(nout_);
 		oval_ = dalloc<float>(nout_);
 		HIPCHECK(hipMemcpyAsync(orow_, off.data(), 4 * ((size_t)Np + 1), hipMemcpyHostToDevice, s));
 		k_outlier_fill<<<gridn(N, kB / 64), kB, 0, s>>>(N, dev.rad.rowptr, dev.rad.col, dev.rad.val, othr_, pinv_,
-		                                                 orow_, ocol_, oval_);
+		                                                 orow_, ocol_, opos_, oval_);
 		HIPCHECK(hipStreamSynchronize(s)); // off lives on this stack
 	}
 	out_built_ = true;
@@ -1539,10 +1614,17 @@ void RadSolver::apply_tiles_f32(const float* xT, float* yT, bool pre)
 	if (part_slots_ < maxslot_)
 		throw std::runtime_error("RadSolver: partial-sum planes fewer than the tile segments need");
 	ensure_perm_colors();
-	k_prep_x32t<<<gridn((uint64_t)kRPad * (Np / 4)), kB, 0, s>>>(xT, dperm_, aperm_, Np, R, pre ? 1 : 0, xq_);
-	if (nchunks_)
-		k_gemm_f32t<<<nblocks_, kB, 0, s>>>(g32t_, xq_, reinterpret_cast<const uint4*>(chunks_), segoff_, tks_, Np,
-		                                     part_);
+	const uint32_t cols = 16 * (uint32_t)col_tiles(R);
+	k_prep_x32t<<<gridn((uint64_t)cols * (Np / 4)), kB, 0, s>>>(xT, dperm_, aperm_, Np, R, cols, pre ? 1 : 0, xq_);
+	if (nchunks_) {
+		const uint4* chs = reinterpret_cast<const uint4*>(chunks_);
+		if (cols == 64)
+			k_gemm_f32t<4><<<nblocks_, kB, 0, s>>>(g32t_, xq_, chs, segoff_, tks_, Np, part_);
+		else if (cols == 128)
+			k_gemm_f32t<8><<<nblocks_, kB, 0, s>>>(g32t_, xq_, chs, segoff_, tks_, Np, part_);
+		else
+			k_gemm_f32t<12><<<nblocks_, kB, 0, s>>>(g32t_, xq_, chs, segoff_, tks_, Np, part_);
+	}
 	k_reduce_split<<<gridn((uint64_t)R * Np), kB, 0, s>>>(part_, 0, nslot_, Np, R, nullptr, 1.0f, yT);
 	HIPCHECK(hipGetLastError());
 }
@@ -1576,8 +1658,10 @@ void RadSolver::apply_dense(int form, const float* xT, float* yT, bool split, bo
 		uint16_t* lo = split ? xqlo_ : nullptr;
 		unsigned* cm = f16 ? cmax_ + cmax_cur_ * kRPad : nullptr;
 		ensure_perm_colors();
-		const unsigned og = (Np / 256) * (kRPad / 16); // k_operand blocks
+		const uint32_t ncg = (R + 15) / 16;
+		const unsigned og = (Np / 256) * ncg; // k_operand blocks
 		OperandPass op;
+		op.ncg = ncg;
 		op.x = xT;
 		op.dperm = dperm_;
 		op.aperm = aperm_;
@@ -1602,22 +1686,37 @@ void RadSolver::apply_dense(int form, const float* xT, float* yT, bool split, bo
 		if (part_slots_ < maxslot_)
 			throw std::runtime_error("RadSolver: partial-sum planes fewer than the tile segments need");
 		if (nchunks_) {
-			const dim3 grid(nblocks_);
 			const uint4* chs = reinterpret_cast<const uint4*>(chunks_);
+			auto gemm = [&](auto p, auto npl, auto nc) {
+				constexpr int P = decltype(p)::value, NPL = decltype(npl)::value, NC = decltype(nc)::value;
+				k_gemm_tiles<P, NPL, ring_depth(NPL, NC), NC><<<nblocks_, kB, 0, s>>>(
+				    g16_, NPL == 2 ? g16lo_ : nullptr, q, NPL == 2 ? lo : nullptr, chs, segoff_, tks_, Np, part_);
+			};
+			auto by_cols = [&](auto p, auto npl) {
+				const int nc = col_tiles(R);
+				if (nc == 4)
+					gemm(p, npl, std::integral_constant<int, 4>{});
+				else if (nc == 8)
+					gemm(p, npl, std::integral_constant<int, 8>{});
+				else
+					gemm(p, npl, std::integral_constant<int, 12>{});
+			};
+			const std::integral_constant<int, 0> bf16;
+			const std::integral_constant<int, 1> fp16, plain;
+			const std::integral_constant<int, 2> comp;
 			if (f16 && split)
-				k_gemm_tiles<1, 2, kTilesD2><<<grid, kB, 0, s>>>(g16_, g16lo_, q, lo, chs, segoff_, tks_, Np, part_);
+				by_cols(fp16, comp);
 			else if (f16)
-				k_gemm_tiles<1, 1, kTilesD1><<<grid, kB, 0, s>>>(g16_, nullptr, q, nullptr, chs, segoff_, tks_, Np,
-				                                                 part_);
+				by_cols(fp16, plain);
 			else if (split)
-				k_gemm_tiles<0, 2, kTilesD2><<<grid, kB, 0, s>>>(g16_, g16lo_, q, lo, chs, segoff_, tks_, Np, part_);
+				by_cols(bf16, comp);
 			else
-				k_gemm_tiles<0, 1, kTilesD1><<<grid, kB, 0, s>>>(g16_, nullptr, q, nullptr, chs, segoff_, tks_, Np,
-				                                                 part_);
+				by_cols(bf16, plain);
 		}
 		// the reduction; chained, it also prepares the next product's operand
 		// (BF16) or the column maxima that scale it (FP16)
 		OperandPass rd;
+		rd.ncg = ncg;
 		rd.part = part_;
 		rd.nslot = nslot_;
 		rd.cmax_in = cm;
@@ -1631,6 +1730,7 @@ void RadSolver::apply_dense(int form, const float* xT, float* yT, bool split, bo
 		if (nout_) {
 			rd.orow = orow_;
 			rd.ocol = ocol_;
+			rd.opos = opos_;
 			rd.oval = oval_;
 			rd.xin = xT;
 		}
