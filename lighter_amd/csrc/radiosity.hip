@@ -1153,29 +1153,70 @@ __global__ __launch_bounds__(kB) void k_gather(uint32_t N, uint32_t R, int logw,
 			}
 }
 
-// layout changes between the row-major (sparse) and column-major (dense) sets
-// (position p holds patch perm[p]; null perm / pinv: the identity)
-template <class A, class B>
-__global__ void k_to_colmajor(const A* __restrict__ x, uint32_t N, uint32_t Np, uint32_t R,
-                              const uint32_t* __restrict__ perm, B* __restrict__ xT)
+// ---------------------------------------------------------------------------
+// Layout changes between the caller's row-major N x R vectors and the
+// column-major sets of the dense and tile forms (position p holds patch
+// perm[p]; null perm: the identity), through LDS tiles of 64 positions x 32
+// columns, so that both sides move in whole runs: element by element the
+// row-major side touched one 8-byte piece of R x 8 bytes per lane.  They are
+// bound by HBM; 32,768 patches, R = 192, 8 bounces: the total in one pass of
+// 100 us (300 MB) instead of 16 passes of 46 and 24 us.
+// ---------------------------------------------------------------------------
+constexpr int kTP = 64, kTC = 32;
+static inline dim3 tile_grid(uint32_t Np, uint32_t R) { return dim3(Np / kTP, (R + kTC - 1) / kTC); }
+
+// columns xT[c][p] = (B)x[perm[p]][c], padding zero
+template <class B>
+__global__ __launch_bounds__(kB) void k_to_cols(const double* __restrict__ x, uint32_t N, uint32_t Np, uint32_t R,
+                                                const uint32_t* __restrict__ perm, B* __restrict__ xT)
 {
-	uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
-	if (t >= (uint64_t)R * Np)
-		return;
-	uint32_t c = (uint32_t)(t / Np), p = (uint32_t)(t % Np);
-	uint32_t j = perm ? perm[p] : p;
-	xT[t] = j < N ? (B)x[(uint64_t)j * R + c] : (B)0;
+	__shared__ B tile[kTP][kTC + 1];
+	const uint32_t p0 = blockIdx.x * kTP, c0 = blockIdx.y * kTC;
+	const uint32_t c = threadIdx.x % kTC, n = threadIdx.x / kTC;
+	for (uint32_t r = n; r < kTP; r += kB / kTC) {
+		const uint32_t j = perm ? perm[p0 + r] : p0 + r;
+		tile[r][c] = j < N && c0 + c < R ? (B)x[(uint64_t)j * R + c0 + c] : (B)0;
+	}
+	__syncthreads();
+	const uint32_t p = threadIdx.x % kTP;
+	for (uint32_t q = threadIdx.x / kTP; q < kTC && c0 + q < R; q += kB / kTP)
+		xT[(uint64_t)(c0 + q) * Np + p0 + p] = tile[p][q];
 }
 
-template <class A, class B>
-__global__ void k_to_rowmajor(const A* __restrict__ xT, uint32_t N, uint32_t Np, uint32_t R,
-                              const uint32_t* __restrict__ pinv, B* __restrict__ x)
+// rows out[perm[p]][c] = x0[perm[p]][c] (0 when x0 is null) + sum_b z[b][c][p],
+// b ascending, in FP64; z: nz column-major sets of zstride elements each
+template <class A>
+__global__ __launch_bounds__(kB) void k_to_rows(const double* __restrict__ x0, const A* __restrict__ z, uint32_t nz,
+                                                uint64_t zstride, uint32_t N, uint32_t Np, uint32_t R,
+                                                const uint32_t* __restrict__ perm, double* __restrict__ out)
 {
-	uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
-	if (t >= (uint64_t)N * R)
-		return;
-	uint32_t j = (uint32_t)(t / R), c = (uint32_t)(t % R);
-	x[t] = (B)xT[(uint64_t)c * Np + (pinv ? pinv[j] : j)];
+	__shared__ double tile[kTP][kTC + 1];
+	const uint32_t p0 = blockIdx.x * kTP, c0 = blockIdx.y * kTC;
+	const uint32_t c = threadIdx.x % kTC, n = threadIdx.x / kTC, p = threadIdx.x % kTP;
+	if (x0)
+		for (uint32_t r = n; r < kTP; r += kB / kTC) {
+			const uint32_t j = perm ? perm[p0 + r] : p0 + r;
+			tile[r][c] = j < N && c0 + c < R ? x0[(uint64_t)j * R + c0 + c] : 0.0;
+		}
+	__syncthreads();
+	for (uint32_t q = threadIdx.x / kTP; q < kTC && c0 + q < R; q += kB / kTP) {
+		const A* src = z + (uint64_t)(c0 + q) * Np + p0 + p;
+		double v = x0 ? tile[p][q] : 0.0;
+		uint32_t b = 0;
+		if (!x0 && nz) { // not 0 + z, which would turn -0 into +0
+			v = (double)src[0];
+			b = 1;
+		}
+		for (; b < nz; ++b)
+			v += (double)src[b * zstride];
+		tile[p][q] = v;
+	}
+	__syncthreads();
+	for (uint32_t r = n; r < kTP; r += kB / kTC) {
+		const uint32_t j = perm ? perm[p0 + r] : p0 + r;
+		if (j < N && c0 + c < R)
+			out[(uint64_t)j * R + c0 + c] = tile[r][c];
+	}
 }
 
 template <class A, class B> __global__ void k_axpy(uint64_t n, const A* __restrict__ x, B* __restrict__ y)
@@ -1183,6 +1224,34 @@ template <class A, class B> __global__ void k_axpy(uint64_t n, const A* __restri
 	uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
 	if (t < n)
 		y[t] += (B)x[t];
+}
+
+// s1 = s0 + z (FP64)
+__global__ void k_partial_sum(uint64_t n, const double* __restrict__ s0, const float* __restrict__ z,
+                              double* __restrict__ s1)
+{
+	const uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
+	if (t < n)
+		s1[t] = s0[t] + (double)z[t];
+}
+
+// k_adj_step on column-major sets (dense and tile forms): column c, position
+// p; diffuse and area in position order (npos of them, the padding's zero);
+// xT receives ybar in FP32, the next product's operand
+__global__ __launch_bounds__(kB) void k_adj_cols(uint32_t Np, uint32_t R, uint32_t npos, const float* __restrict__ u,
+                                                 const double* __restrict__ sprev, const float* __restrict__ diffuse,
+                                                 const float* __restrict__ area, double* __restrict__ dalb,
+                                                 double* __restrict__ lam, float* __restrict__ xT)
+{
+	const uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
+	if (t >= (uint64_t)R * Np)
+		return;
+	const uint32_t c = (uint32_t)(t / Np), p = (uint32_t)(t % Np);
+	const double au = (p < npos ? (double)area[p] : 0.0) * (double)u[t];
+	dalb[t] += au * sprev[t];
+	const double yb = (p < npos ? (double)diffuse[3 * p + c % 3] : 0.0) * au;
+	lam[t] += yb;
+	xT[t] = (float)yb;
 }
 
 // one step of the adjoint sweep (row-major N x R, FP64), with u = H ybar_k:
@@ -1278,8 +1347,8 @@ void RadSolver::release()
 	dfree(part_);
 	dfree(xq_);
 	dfree(xqlo_);
-	dfree(xT_);
-	dfree(yT_);
+	dfree(keep32_);
+	dfree(keep64_);
 	dfree(rmx_);
 	dfree(rmx64_);
 	dfree(cmax_);
@@ -1302,13 +1371,17 @@ void RadSolver::set_problem(const double* E, uint32_t R_, const float* diffuse3,
 	}
 	R = R_;
 	hipStream_t s = (hipStream_t)s_;
-	dfree(E_);
-	dfree(diff_);
-	dfree(area_);
 	pcol_ok_ = false;
-	E_ = dalloc<double>((size_t)N * R);
-	diff_ = dalloc<float>(3 * (size_t)N);
-	area_ = dalloc<float>((size_t)Np);
+	if ((uint64_t)N * R > E_n_) {
+		dfree(E_);
+		E_n_ = 0;
+		E_ = dalloc<double>((size_t)N * R);
+		E_n_ = (uint64_t)N * R;
+	}
+	if (!diff_) {
+		diff_ = dalloc<float>(3 * (size_t)N);
+		area_ = dalloc<float>((size_t)Np);
+	}
 	HIPCHECK(hipMemcpyAsync(E_, E, 8 * (size_t)N * R, hipMemcpyHostToDevice, s));
 	HIPCHECK(hipMemcpyAsync(diff_, diffuse3, 12 * (size_t)N, hipMemcpyHostToDevice, s));
 	HIPCHECK(hipMemsetAsync(area_, 0, 4 * (size_t)Np, s));
@@ -1582,8 +1655,6 @@ void RadSolver::ensure_work(int form)
 	if (form >= kDenseF32 && !xq_) {
 		xq_ = dalloc<float>(n); // FP32 operand, or the 16-bit one in its first half
 		xqlo_ = dalloc<uint16_t>(n);
-		xT_ = dalloc<float>(n);
-		yT_ = dalloc<float>(n);
 		cmax_ = dalloc<unsigned>(2 * kRPad);
 	}
 	if (form == kSparseF32 && !rmx_)
@@ -1754,44 +1825,59 @@ void RadSolver::apply_dense(int form, const float* xT, float* yT, bool split, bo
 	HIPCHECK(hipGetLastError());
 }
 
-// y = K x (pre) or H x, row-major N x R FP64 in and out, in the given form;
-// tot += y when tot is given
-void RadSolver::apply_op(int form, const double* x, double* y, bool pre, double* tot)
+// y = K x (pre) or H x over the links, row-major N x R FP64 in and out, in the
+// given sparse form; tot += y when tot is given
+void RadSolver::apply_sparse(int form, const double* x, double* y, bool pre, double* tot)
 {
 	hipStream_t s = (hipStream_t)s_;
-	const uint64_t nR = (uint64_t)N * R, nRp = (uint64_t)R * Np;
+	const uint64_t nR = (uint64_t)N * R;
 	const unsigned sgrid = gridn(N, kB / 64);
 	const uint32_t* rp = dev.rad.rowptr;
 	const uint32_t* cl = dev.rad.col;
 	const float* vl = dev.rad.val;
-	if (form == kSparseF64 || form == kSparseF32) {
-		auto product = [&](auto* xp) {
-			using T = std::remove_pointer_t<decltype(xp)>;
-			if (pre)
-				k_prep_rows<T, true><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, xp);
-			else
-				k_prep_rows<T, false><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, xp);
-			int logw = 0;
-			while (logw < 6 && (1u << logw) < R)
-				++logw;
-			if (R <= 64)
-				k_gather<T, 1><<<sgrid, kB, 0, s>>>(N, R, logw, rp, cl, vl, xp, y, tot);
-			else
-				k_gather<T, 3><<<sgrid, kB, 0, s>>>(N, R, logw, rp, cl, vl, xp, y, tot);
-		};
-		if (form == kSparseF64)
-			product(rmx64_);
+	auto product = [&](auto* xp) {
+		using T = std::remove_pointer_t<decltype(xp)>;
+		if (pre)
+			k_prep_rows<T, true><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, xp);
 		else
-			product(rmx_);
-	} else {
-		const bool mo = storage_of(form) != kDenseF32; // Morton order
-		k_to_colmajor<double, float><<<gridn(nRp), kB, 0, s>>>(x, N, Np, R, mo ? perm_ : nullptr, xT_);
-		apply_dense(form, xT_, yT_, false, pre);
-		k_to_rowmajor<float, double><<<gridn(nR), kB, 0, s>>>(yT_, N, Np, R, mo ? pinv_ : nullptr, y);
-		if (tot)
-			k_axpy<double, double><<<gridn(nR), kB, 0, s>>>(nR, y, tot);
-	}
+			k_prep_rows<T, false><<<gridn(nR), kB, 0, s>>>(nR, R, x, diff_, area_, xp);
+		int logw = 0;
+		while (logw < 6 && (1u << logw) < R)
+			++logw;
+		if (R <= 64)
+			k_gather<T, 1><<<sgrid, kB, 0, s>>>(N, R, logw, rp, cl, vl, xp, y, tot);
+		else
+			k_gather<T, 3><<<sgrid, kB, 0, s>>>(N, R, logw, rp, cl, vl, xp, y, tot);
+	};
+	if (form == kSparseF64)
+		product(rmx64_);
+	else
+		product(rmx_);
 	HIPCHECK(hipGetLastError());
+}
+
+// n doubles (n floats of the iterates) kept across calls: allocating and
+// freeing them on every call cost more than a small problem's products.
+double* RadSolver::keep64(uint64_t n)
+{
+	if (n > keep64_n_) {
+		dfree(keep64_);
+		keep64_n_ = 0;
+		keep64_ = dalloc<double>(n);
+		keep64_n_ = n;
+	}
+	return keep64_;
+}
+
+float* RadSolver::keep32(uint64_t n)
+{
+	if (n > keep32_n_) {
+		dfree(keep32_);
+		keep32_n_ = 0;
+		keep32_ = dalloc<float>(n);
+		keep32_n_ = n;
+	}
+	return keep32_;
 }
 
 void RadSolver::solve(int form, int bounces, int refine, double* total_out)
@@ -1802,19 +1888,19 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 	if (refine > 0 && form != kDenseBF16 && form != kDenseF16)
 		throw std::runtime_error("RadSolver: refinement sweeps apply to the plain 16-bit forms (3, 4)");
 	hipStream_t s = (hipStream_t)s_;
-	uint64_t nR = (uint64_t)N * R, nRp = (uint64_t)R * Np;
+	const uint64_t nR = (uint64_t)N * R, nRp = (uint64_t)R * Np;
 	times = RadTimes{};
 	ensure_work(form);
-	// FP64 running total
-	DevBuf<double> tot(nR);
-	HIPCHECK(hipMemcpyAsync(tot, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
+	double* tot = keep64((form < kDenseF32 ? 3 : 1) * nR); // FP64 total
 	if (form == kSparseF64 || form == kSparseF32) {
-		DevBuf<double> x(nR), y(nR);
-		HIPCHECK(hipMemcpyAsync(x, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
+		HIPCHECK(hipMemcpyAsync(tot, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
+		const double* x = E_;
+		double *y = tot + nR, *y2 = tot + 2 * nR;
 		Ev ev(s);
 		for (int b = 0; b < bounces; ++b) {
-			apply_op(form, x, y, true, tot);
-			std::swap(x, y);
+			apply_sparse(form, x, y, true, tot);
+			x = y;
+			std::swap(y, y2);
 		}
 		times.series_ms = ev.stop();
 		times.per_bounce_ms = times.series_ms / std::max(1, bounces);
@@ -1823,14 +1909,13 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 			build_dense(form);
 		times.build_ms = build_ms;
 		// z_k (column-major FP32), k = 0..b
-		std::vector<DevBuf<float>> z;
+		float* z0 = keep32((uint64_t)(bounces + 1) * nRp);
+		std::vector<float*> z;
 		for (int b = 0; b <= bounces; ++b)
-			z.emplace_back(nRp);
+			z.push_back(z0 + (uint64_t)b * nRp);
 		// the tile forms keep z in Morton order
-		const bool mo = storage_of(form) != kDenseF32;
-		const uint32_t* po = mo ? perm_ : nullptr;
-		const uint32_t* pi = mo ? pinv_ : nullptr;
-		k_to_colmajor<double, float><<<gridn(nRp), kB, 0, s>>>(E_, N, Np, R, po, z[0]);
+		const uint32_t* po = storage_of(form) != kDenseF32 ? perm_ : nullptr;
+		k_to_cols<float><<<tile_grid(Np, R), kB, 0, s>>>(E_, N, Np, R, po, z0);
 		{
 			Ev ev(s);
 			for (int b = 1; b <= bounces; ++b)
@@ -1844,7 +1929,6 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 		// the difference taken in FP64; corrections d_b = Kdense d_{b-1} + rho_b
 		// (d_0 = 0: z_0 = E is exact) with the plain 16-bit product; then
 		// z += d.  z_{b-1} is corrected only after rho_b has used its old value.
-		DevBuf<double> zr(nR);
 		if (refine > 0) {
 			DevBuf<double> rho(nRp);
 			DevBuf<float> kz(nRp), d(nRp), dprev(nRp);
@@ -1865,10 +1949,7 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 		}
 		HIPCHECK(hipGetLastError());
 		// total = sum_k z_k in FP64 (z_0 = E exactly)
-		for (int b = 1; b <= bounces; ++b) {
-			k_to_rowmajor<float, double><<<gridn(nR), kB, 0, s>>>(z[b], N, Np, R, pi, zr);
-			k_axpy<double, double><<<gridn(nR), kB, 0, s>>>(nR, zr, tot);
-		}
+		k_to_rows<float><<<tile_grid(Np, R), kB, 0, s>>>(E_, z0 + nRp, (uint32_t)bounces, nRp, N, Np, R, po, tot);
 	}
 	HIPCHECK(hipGetLastError());
 	HIPCHECK(hipMemcpyAsync(total_out, tot, 8 * nR, hipMemcpyDeviceToHost, s));
@@ -1897,19 +1978,25 @@ void RadSolver::solve_grad(int form, int bounces, const double* g, double* total
 	if (form >= kDenseF32 && built_form_ != storage_of(form))
 		build_dense(form);
 	const int B = std::max(0, bounces);
-	std::vector<DevBuf<double>> S;
-	for (int k = 0; k < std::max(1, B); ++k)
-		S.emplace_back(nR);
-	DevBuf<double> z(nR), zn(nR), tot(nR), ybar(nR), u(nR), lam(nR), dalb(nR);
+	if (form >= kDenseF32) {
+		grad_dense(form, B, g, total_out, lam_out, dalb_out);
+		return;
+	}
+	// row-major N x R sets: S_0 .. S_{B-1}, then the vectors of the sweeps
+	const uint64_t nS = std::max(1, B);
+	double* S = keep64((nS + 7) * nR);
+	double *z = S + nS * nR, *zn = z + nR, *tot = zn + nR, *ybar = tot + nR, *u = ybar + nR, *lam = u + nR,
+	       *dalb = lam + nR;
 	Ev ev(s);
 	// forward: S_0 = E, z_k = K z_{k-1}, S_k = S_{k-1} + z_k
-	HIPCHECK(hipMemcpyAsync(S[0], E_, 8 * nR, hipMemcpyDeviceToDevice, s));
-	HIPCHECK(hipMemcpyAsync(z, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
+	HIPCHECK(hipMemcpyAsync(S, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
 	HIPCHECK(hipMemcpyAsync(tot, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
+	const double* x = E_;
 	for (int k = 1; k <= B; ++k) {
-		apply_op(form, z, zn, true, tot);
+		apply_sparse(form, x, zn, true, tot);
 		if (k < B)
-			HIPCHECK(hipMemcpyAsync(S[k], tot, 8 * nR, hipMemcpyDeviceToDevice, s));
+			HIPCHECK(hipMemcpyAsync(S + k * nR, tot, 8 * nR, hipMemcpyDeviceToDevice, s));
+		x = zn;
 		std::swap(z, zn);
 	}
 	times.series_ms = ev.stop();
@@ -1919,8 +2006,8 @@ void RadSolver::solve_grad(int form, int bounces, const double* g, double* total
 	HIPCHECK(hipMemcpyAsync(lam, ybar, 8 * nR, hipMemcpyDeviceToDevice, s));
 	HIPCHECK(hipMemsetAsync(dalb, 0, 8 * nR, s));
 	for (int k = B; k >= 1; --k) {
-		apply_op(form, ybar, u, false);
-		k_adj_step<<<gridn(nR), kB, 0, s>>>(N, R, u, S[k - 1], diff_, area_, dalb, ybar, lam);
+		apply_sparse(form, ybar, u, false);
+		k_adj_step<<<gridn(nR), kB, 0, s>>>(N, R, u, S + (k - 1) * nR, diff_, area_, dalb, ybar, lam);
 	}
 	times.refine_ms = ev2.stop(); // the reverse sweep's time
 	times.per_bounce_ms = times.refine_ms / std::max(1, B);
@@ -1928,6 +2015,55 @@ void RadSolver::solve_grad(int form, int bounces, const double* g, double* total
 	HIPCHECK(hipMemcpyAsync(total_out, tot, 8 * nR, hipMemcpyDeviceToHost, s));
 	HIPCHECK(hipMemcpyAsync(lam_out, lam, 8 * nR, hipMemcpyDeviceToHost, s));
 	HIPCHECK(hipMemcpyAsync(dalb_out, dalb, 8 * nR, hipMemcpyDeviceToHost, s));
+	HIPCHECK(hipStreamSynchronize(s));
+}
+
+// The same for the dense and tile forms, every vector column-major in the
+// product's own position order: the iterates stay where the products read
+// and write them, and the caller's rows are transposed once on entry and
+// once per result.
+void RadSolver::grad_dense(int form, int B, const double* g, double* total_out, double* lam_out, double* dalb_out)
+{
+	hipStream_t s = (hipStream_t)s_;
+	const uint64_t nR = (uint64_t)N * R, nRp = (uint64_t)R * Np;
+	const bool mo = storage_of(form) != kDenseF32; // Morton order
+	const uint32_t* po = mo ? perm_ : nullptr;
+	const dim3 tg = tile_grid(Np, R);
+	if (mo)
+		ensure_perm_colors();
+	const float* diff = mo ? dperm_ : diff_;
+	const float* area = mo ? aperm_ : area_;
+	const uint32_t npos = mo ? Np : N;
+	double* S = keep64((uint64_t)(B + 3) * nRp + nR); // S_0 .. S_B, dalb, lam, then rows of the caller
+	double *dalb = S + (uint64_t)(B + 1) * nRp, *lam = dalb + nRp, *rows = lam + nRp;
+	float *z = keep32(2 * nRp), *zn = z + nRp;
+	Ev ev(s);
+	// forward: S_0 = E, z_k = K z_{k-1}, S_k = S_{k-1} + z_k
+	k_to_cols<double><<<tg, kB, 0, s>>>(E_, N, Np, R, po, S);
+	k_to_cols<float><<<tg, kB, 0, s>>>(E_, N, Np, R, po, z);
+	for (int k = 1; k <= B; ++k) {
+		apply_dense(form, z, zn, false, true, k < B);
+		k_partial_sum<<<gridn(nRp), kB, 0, s>>>(nRp, S + (k - 1) * nRp, zn, S + k * nRp);
+		std::swap(z, zn);
+	}
+	times.series_ms = ev.stop();
+	// reverse sweep
+	Ev ev2(s);
+	HIPCHECK(hipMemcpyAsync(rows, g, 8 * nR, hipMemcpyHostToDevice, s));
+	k_to_cols<double><<<tg, kB, 0, s>>>(rows, N, Np, R, po, lam);
+	k_to_cols<float><<<tg, kB, 0, s>>>(rows, N, Np, R, po, z);
+	HIPCHECK(hipMemsetAsync(dalb, 0, 8 * nRp, s));
+	for (int k = B; k >= 1; --k) {
+		apply_dense(form, z, zn, false, false);
+		k_adj_cols<<<gridn(nRp), kB, 0, s>>>(Np, R, npos, zn, S + (k - 1) * nRp, diff, area, dalb, lam, z);
+	}
+	times.refine_ms = ev2.stop(); // the reverse sweep's time
+	times.per_bounce_ms = times.refine_ms / std::max(1, B);
+	for (auto [src, out] : {std::pair<double*, double*>{S + B * nRp, total_out}, {lam, lam_out}, {dalb, dalb_out}}) {
+		k_to_rows<double><<<tg, kB, 0, s>>>(nullptr, src, 1, nRp, N, Np, R, po, rows);
+		HIPCHECK(hipGetLastError());
+		HIPCHECK(hipMemcpyAsync(out, rows, 8 * nR, hipMemcpyDeviceToHost, s));
+	}
 	HIPCHECK(hipStreamSynchronize(s));
 }
 
