@@ -204,16 +204,15 @@ LTRAPI int lgx_AmbientOcclusion(lgx_Device* dev, const float* randoff, int num_s
                                 float multiplier, float falloff, float effect, const float* color3);
 /* Radiosity links among N patches (Int_RDGenLinks pair loop,
  * lighter.cpp:728-759); returns the link count through nlinks.  The pairs
- * are found on a uniform grid of cells as wide as the longest distance a
- * pair can link over (f >= 0.001 needs l^2 <= |nA| |nB| / (0.001 pi)), so
- * any patch count whose links fit 2^32 CSR entries is taken; with
- * non-finite positions or normals the search falls back to all pairs. */
+ * are found among clusters of 64 neighbouring patches whose positions and
+ * normals allow a factor of 0.001 between them, so any patch count whose
+ * links fit 2^32 CSR entries is taken; with non-finite positions or normals
+ * the search falls back to all pairs. */
 LTRAPI int lgx_RadLinks(lgx_Device* dev, const float* pos3, const float* nrm3, size_t n, size_t* nlinks);
 /* No counterpart in the reference (tests). How the next lgx_RadLinks
- * finds its candidate pairs: mode 0 (default) the grid, unless it would
- * test more than N^2 / 4 pairs (a scene within one cell width), then all
- * pairs; 1 all pairs, as the reference's loop does (at most 524,288
- * patches); 2 the grid.  Every mode gives the same links. */
+ * finds its candidate pairs: modes 0 (default) and 2 among clusters of
+ * patches, mode 1 all pairs, as the reference's loop does (at most 524,288
+ * patches).  Every mode gives the same links. */
 LTRAPI int lgx_SetLinkSearch(lgx_Device* dev, int mode);
 LTRAPI int lgx_RadReadLinks(lgx_Device* dev, uint32_t* rowmap, uint32_t* other, float* factor);
 /* bounce_count rounds of Int_RDBounce (lighter.cpp:767-797) from emitted

@@ -164,12 +164,11 @@ public:
 	// Patches = samples.  rad_links builds the symmetric link structure of
 	// the pairs that pass the form-factor thresholds and whose segment hits
 	// a shadow caster (the reference's VisibilityTest returns the hit).
-	// Candidates come from a uniform grid of cells as wide as the longest
-	// distance a pair can link over, or from all pairs as the reference
-	// enumerates them (at most kMaxAllPairsPatches patches); both give the
-	// same links.  links_mode 0: the grid, unless it would test more than
-	// N^2 / 4 pairs (then all pairs); 1: all pairs; 2: the grid.  Patches
-	// with non-finite positions or normals always take all pairs.
+	// Candidates come from pairs of clusters of patches whose bounds allow a
+	// link, or from all pairs as the reference enumerates them (at most
+	// kMaxAllPairsPatches patches); both give the same links.  links_mode 0
+	// and 2: the clusters; 1: all pairs.  Patches with non-finite positions
+	// or normals always take all pairs.
 	void rad_set_patches(const float* pos, const float* nrm, size_t n);
 	size_t rad_links();
 	int links_mode = 0;
@@ -250,7 +249,8 @@ private:
 	// candidate pairs (uint2, i < j, device memory), grouped by row i;
 	// coff (N + 1, device) receives the first candidate of each row
 	void* link_candidates_all(uint64_t& ncand, uint64_t* coff);
-	void* link_candidates_grid(uint64_t& ncand, uint64_t* coff); // the same set from the grid
+	uint64_t links_by_all_pairs(uint32_t** colx); // CSR entries; the unsorted columns
+	uint64_t links_by_clusters(uint32_t** colx);
 	size_t nsamples_ = 0;
 	// direct light
 	float* d_w_ = nullptr;

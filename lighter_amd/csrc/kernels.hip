@@ -1657,112 +1657,454 @@ __global__ __launch_bounds__(kBlock) void k_pairs(const float* __restrict__ pos,
 }
 
 // ---------------------------------------------------------------------------
-// Link candidates over a uniform grid of the patches.  A pair passes the
-// factor thresholds only when f = dA dB / (pi l^4) >= kSmall, and dA, dB <=
-// |n| l, so l^2 <= |nA| |nB| / (pi kSmall): 17.8 m for unit normals.  With
-// cells at least that wide every pair that can pass lies in the same or a
-// neighbouring cell; those pairs are tested with the arithmetic of the
-// all-pairs search (pair_factor, the lower index as A), so both searches
-// find the same candidate set, in another order.
+// The link search over clusters of 64 patches.  Patches are binned by the
+// dominant axis of their normal and a cell of their position, so a cluster
+// (and each quarter of it) is a compact patch of one kind of surface; its box
+// and the range of its normals bound every factor between two clusters, and
+// only pairs of clusters with quarters that could hold a pair of kSmall or
+// more are looked at.  One wave takes a pair of clusters and tests its pairs
+// of patches with the arithmetic of the all-pairs search (pair_factor; it
+// gives the same bits from either end, since the differences and dot
+// products only change sign) into a 64 x 64 bit matrix; the occlusion tests
+// take 64 of its pairs at a time, which start and end at neighbouring
+// patches, and leave the links' bits in it.  No candidate is stored, and the
+// CSR's counts and cursors take one atomic per patch and cluster pair
+// instead of one per link.
 // ---------------------------------------------------------------------------
-struct LinkGrid {
-	float lo[3];
-	float inv;     // 1 / cell width
-	uint32_t n[3]; // cells per axis (product below 2^24)
-	int reach;     // cells searched on each side: the cells are 1 / reach of the linking distance wide
+constexpr uint32_t kCl = 64;        // patches per cluster, and clusters per super-cluster
+constexpr uint32_t kNoPatch = ~0u;  // padding of the last cluster
+
+struct ClBox {
+	float lo[3], hi[3];   // positions
+	float nlo[3], nhi[3]; // normals
 };
 
-__device__ __forceinline__ uint32_t grid_cell(const LinkGrid& G, f3 p)
+// Bins of the patches: the dominant axis and sign of the normal, then the
+// cell of a uniform grid along a Morton curve (in x-major order the 64
+// patches of a cluster lay in a row of cells, 119 m long in a city).
+struct PatchBins {
+	float lo[3], inv;  // 1 / cell width
+	uint32_t bits[3];  // 2^bits cells per axis
+};
+
+__global__ void k_patch_bins(const float* __restrict__ pos, const float* __restrict__ nrm, uint32_t N, PatchBins G,
+                             uint32_t* __restrict__ bin, uint32_t* __restrict__ count)
 {
+	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= N)
+		return;
+	const f3 p = ld3(pos + 3 * (size_t)i), n = ld3(nrm + 3 * (size_t)i);
+	const float ax = fabsf(n.x), ay = fabsf(n.y), az = fabsf(n.z);
+	const uint32_t side = ax >= ay && ax >= az ? (n.x < 0 ? 0u : 1u) : ay >= az ? (n.y < 0 ? 2u : 3u) : (n.z < 0 ? 4u : 5u);
 	const float q[3] = {(p.x - G.lo[0]) * G.inv, (p.y - G.lo[1]) * G.inv, (p.z - G.lo[2]) * G.inv};
-	uint32_t c[3];
-#pragma unroll
+	uint32_t c[3], k = side, bits = max(max(G.bits[0], G.bits[1]), G.bits[2]);
 	for (int a = 0; a < 3; ++a)
-		c[a] = min(G.n[a] - 1, (uint32_t)floorf(q[a])); // p >= lo: q >= 0
-	return (c[2] * G.n[1] + c[1]) * G.n[0] + c[0];
+		c[a] = min((1u << G.bits[a]) - 1, (uint32_t)q[a]); // p >= lo: q >= 0
+	while (bits--)
+		for (int a = 2; a >= 0; --a)
+			if (bits < G.bits[a])
+				k = k << 1 | (c[a] >> bits & 1u);
+	bin[i] = k;
+	atomicAdd(count + k, 1u);
 }
 
-__global__ void k_grid_count(const float* __restrict__ pos, uint32_t N, LinkGrid G, uint32_t* __restrict__ cell,
-                             uint32_t* __restrict__ ccount)
+// The patches in bin order (any order within a bin: it only decides which
+// patches share a cluster), padded to whole clusters: position and index,
+// normal.  count serves as the bins' cursors, counted down to zero.
+__global__ void k_patch_place(const float* __restrict__ pos, const float* __restrict__ nrm, uint32_t N, uint32_t Npad,
+                              const uint32_t* __restrict__ bin, const uint64_t* __restrict__ start,
+                              uint32_t* __restrict__ count, float4* __restrict__ sp, float4* __restrict__ sn)
 {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= N)
+	if (i >= Npad)
 		return;
-	const uint32_t k = grid_cell(G, ld3(pos + 3 * i));
-	cell[i] = k;
-	atomicAdd(ccount + k, 1u);
+	uint64_t t = i;
+	float4 a = make_float4(0, 0, 0, __uint_as_float(kNoPatch)), b = make_float4(0, 0, 0, 0);
+	if (i < N) {
+		const uint32_t k = bin[i];
+		t = start[k] + (atomicSub(count + k, 1u) - 1u);
+		const f3 p = ld3(pos + 3 * (size_t)i), n = ld3(nrm + 3 * (size_t)i);
+		a = make_float4(p.x, p.y, p.z, __uint_as_float(i));
+		b = make_float4(n.x, n.y, n.z, 0.0f);
+	}
+	sp[t] = a;
+	sn[t] = b;
 }
 
-__global__ void k_grid_fill(uint32_t N, const uint32_t* __restrict__ cell, const uint64_t* __restrict__ cstart,
-                            uint32_t* __restrict__ cfill, uint32_t* __restrict__ order)
+// the union over the lane's group of G lanes
+template <int G>
+__device__ __forceinline__ void group_box(ClBox& b)
 {
-	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= N)
-		return;
-	const uint32_t k = cell[i];
-	order[cstart[k] + atomicAdd(cfill + k, 1u)] = i;
+	for (int o = G / 2; o > 0; o >>= 1)
+		for (int a = 0; a < 3; ++a) {
+			b.lo[a] = fminf(b.lo[a], __shfl_xor(b.lo[a], o));
+			b.hi[a] = fmaxf(b.hi[a], __shfl_xor(b.hi[a], o));
+			b.nlo[a] = fminf(b.nlo[a], __shfl_xor(b.nlo[a], o));
+			b.nhi[a] = fmaxf(b.nhi[a], __shfl_xor(b.nhi[a], o));
+		}
 }
 
-// Pass 0 counts, pass 1 writes the candidates (i, j > i) of row i from the
-// (2 reach + 1)^3 cells around i's cell; thread t takes the t-th patch in
-// cell order.
+__device__ __forceinline__ ClBox empty_box()
+{
+	ClBox b;
+	for (int a = 0; a < 3; ++a) {
+		b.lo[a] = b.nlo[a] = INFINITY;
+		b.hi[a] = b.nhi[a] = -INFINITY;
+	}
+	return b;
+}
+
+// one wave per cluster: its bounds and those of its quarters (16 patches)
+__global__ __launch_bounds__(kBlock) void k_cluster_boxes(const float4* __restrict__ sp, const float4* __restrict__ sn,
+                                                          uint32_t nc, ClBox* __restrict__ box, ClBox* __restrict__ quart)
+{
+	const uint32_t c = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+	if (c >= nc)
+		return;
+	ClBox b = empty_box();
+	const float4 p = sp[(size_t)c * kCl + lane], n = sn[(size_t)c * kCl + lane];
+	if (__float_as_uint(p.w) != kNoPatch) {
+		b.lo[0] = b.hi[0] = p.x, b.lo[1] = b.hi[1] = p.y, b.lo[2] = b.hi[2] = p.z;
+		b.nlo[0] = b.nhi[0] = n.x, b.nlo[1] = b.nhi[1] = n.y, b.nlo[2] = b.nhi[2] = n.z;
+	}
+	group_box<16>(b);
+	if ((lane & 15) == 0)
+		quart[4 * (size_t)c + (lane >> 4)] = b;
+	group_box<64>(b);
+	if (lane == 0)
+		box[c] = b;
+}
+
+// one wave per super-cluster: the bounds of its 64 clusters
+__global__ __launch_bounds__(kBlock) void k_super_boxes(const ClBox* __restrict__ box, uint32_t nc, uint32_t ns,
+                                                        ClBox* __restrict__ sup)
+{
+	const uint32_t s = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+	if (s >= ns)
+		return;
+	const size_t c = (size_t)s * kCl + lane;
+	ClBox b = c < nc ? box[c] : empty_box();
+	group_box<64>(b);
+	if (lane == 0)
+		sup[s] = b;
+}
+
+// False when no patch of A and patch of B can pass pair_factor.  With d
+// from A to B in [dlo, dhi], dA = nA . d and dB = -nB . d are at most the
+// interval products' sums; both have to exceed kSmall, and f = dA dB / (pi
+// l^4) has to reach it with l at least the boxes' distance; dA <= |nA| l and
+// dB <= |nB| l give three more bounds.  The margins (4e-6 of the terms'
+// magnitude, 1e-3 of f) are tens of times the rounding of pair_factor and of
+// these bounds.  Distances of 1e9 and more, whose powers might overflow in
+// pair_factor, are left to it.
+__device__ __forceinline__ bool may_link(const ClBox& A, const ClBox& B)
+{
+	float da = 0, db = 0, l2 = 0, ext = 0, na = 0, nb = 0, na2 = 0, nb2 = 0;
+#pragma unroll
+	for (int a = 0; a < 3; ++a) {
+		const float dlo = B.lo[a] - A.hi[a], dhi = B.hi[a] - A.lo[a];
+		da += fmaxf(fmaxf(A.nlo[a] * dlo, A.nlo[a] * dhi), fmaxf(A.nhi[a] * dlo, A.nhi[a] * dhi));
+		db += fmaxf(fmaxf(-B.nlo[a] * dlo, -B.nlo[a] * dhi), fmaxf(-B.nhi[a] * dlo, -B.nhi[a] * dhi));
+		const float gap = fmaxf(fmaxf(dlo, -dhi), 0.0f);
+		l2 += gap * gap;
+		ext += fmaxf(fabsf(dlo), fabsf(dhi));
+		const float ma = fmaxf(fabsf(A.nlo[a]), fabsf(A.nhi[a])), mb = fmaxf(fabsf(B.nlo[a]), fabsf(B.nhi[a]));
+		na += ma;
+		nb += mb;
+		na2 += ma * ma;
+		nb2 += mb * mb;
+	}
+	da += 4e-6f * ext * na;
+	db += 4e-6f * ext * nb;
+	if (da <= kSmall || db <= kSmall)
+		return false;
+	if (l2 > 0.0f && l2 < 1e18f) {
+		const float l = sqrtf(l2), lim = kSmall * kPiF * 0.999f;
+		na2 = sqrtf(na2) * 1.0001f;
+		nb2 = sqrtf(nb2) * 1.0001f;
+		if (da * db < lim * l2 * l2 || da * nb2 < lim * l2 * l || db * na2 < lim * l2 * l || na2 * nb2 < lim * l2)
+			return false;
+	}
+	return true;
+}
+
+// One wave per cluster a: its partners b >= a, super-clusters first, then
+// clusters, then the 16 pairs of quarters (four partners at a time).  Pass 0
+// counts, pass 1 writes the pair and the quarters that may link (bit 4 qa +
+// qb).
 template <bool WRITE>
-__global__ __launch_bounds__(kBlock) void k_pairs_grid(const float* __restrict__ pos, const float* __restrict__ nrm,
-                                                       uint32_t N, LinkGrid G, const uint32_t* __restrict__ cell,
-                                                       const uint64_t* __restrict__ cstart,
-                                                       const uint32_t* __restrict__ order,
-                                                       uint32_t* __restrict__ counts,
-                                                       const uint64_t* __restrict__ offs, uint2* __restrict__ cand)
+__global__ __launch_bounds__(kBlock) void k_cluster_pairs(const ClBox* __restrict__ box, const ClBox* __restrict__ quart,
+                                                          uint32_t nc, const ClBox* __restrict__ sup, uint32_t ns,
+                                                          uint32_t* __restrict__ count,
+                                                          const uint64_t* __restrict__ offs, uint2* __restrict__ out,
+                                                          uint16_t* __restrict__ quarters)
 {
-	const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= N)
+	const uint32_t a = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+	if (a >= nc)
 		return;
-	const uint32_t i = order[t]; // neighbouring lanes share cells: they walk the same lists
-	const uint32_t k = cell[i];
-	const int cx = (int)(k % G.n[0]), cy = (int)((k / G.n[0]) % G.n[1]), cz = (int)(k / (G.n[0] * G.n[1]));
-	const f3 ap = ld3(pos + 3 * i), an = ld3(nrm + 3 * i);
-	uint32_t n = 0;
-	const uint64_t base = WRITE ? offs[i] : 0;
-	const int q = G.reach;
-	for (int z = max(cz - q, 0); z <= min(cz + q, (int)G.n[2] - 1); ++z)
-		for (int y = max(cy - q, 0); y <= min(cy + q, (int)G.n[1] - 1); ++y)
-			for (int x = max(cx - q, 0); x <= min(cx + q, (int)G.n[0] - 1); ++x) {
-				const uint32_t cc = ((uint32_t)z * G.n[1] + (uint32_t)y) * G.n[0] + (uint32_t)x;
-				const uint64_t e = cstart[cc + 1];
-				uint64_t q = cstart[cc];
-				// four patches per round: their loads are in flight together
-				for (; q + 4 <= e; q += 4) {
-					uint32_t j[4];
-					f3 bp[4], bn[4];
-#pragma unroll
-					for (int u = 0; u < 4; ++u)
-						j[u] = order[q + u];
-#pragma unroll
-					for (int u = 0; u < 4; ++u) {
-						bp[u] = ld3(pos + 3 * j[u]);
-						bn[u] = ld3(nrm + 3 * j[u]);
-					}
-#pragma unroll
-					for (int u = 0; u < 4; ++u)
-						if (j[u] > i && !(pair_factor(ap, an, bp[u], bn[u]) < 0.0f)) {
-							if (WRITE)
-								cand[base + n] = make_uint2(i, j[u]);
-							n++;
-						}
+	const ClBox A = box[a], Aq = quart[4 * (size_t)a + ((lane >> 2) & 3)];
+	uint64_t at = WRITE ? offs[a] : 0;
+	for (uint32_t s0 = a / kCl; s0 < ns; s0 += 64) {
+		uint64_t m = __ballot(s0 + lane < ns && may_link(A, sup[min(s0 + lane, ns - 1)]));
+		while (m) {
+			const uint32_t b0 = (s0 + (uint32_t)__ffsll((unsigned long long)m) - 1u) * kCl, b = b0 + lane;
+			m &= m - 1;
+			uint64_t k = __ballot(b >= a && b < nc && may_link(A, box[min(b, nc - 1)]));
+			while (k) {
+				// the next four partners, one per 16 lanes
+				uint32_t mine = 64;
+				for (uint32_t g = 0; g < 4 && k; ++g) {
+					if (lane >> 4 == g)
+						mine = (uint32_t)__ffsll((unsigned long long)k) - 1u;
+					k &= k - 1;
 				}
-				for (; q < e; ++q) {
-					const uint32_t j = order[q];
-					if (j <= i)
+				const bool ok = mine < 64 && may_link(Aq, quart[4 * (size_t)(b0 + (mine & 63)) + (lane & 3)]);
+				const uint64_t q = __ballot(ok);
+				for (uint32_t g = 0; g < 4; ++g) {
+					const uint32_t bits = (uint32_t)(q >> (16 * g)) & 0xffffu;
+					if (!bits)
 						continue;
-					if (!(pair_factor(ap, an, ld3(pos + 3 * j), ld3(nrm + 3 * j)) < 0.0f)) {
-						if (WRITE)
-							cand[base + n] = make_uint2(i, j);
-						n++;
+					if (WRITE && lane == 16 * g) {
+						out[at] = make_uint2(a, b0 + mine);
+						quarters[at] = (uint16_t)bits;
 					}
+					++at;
 				}
 			}
-	if (!WRITE)
-		counts[i] = n;
+		}
+	}
+	if (!WRITE && lane == 0)
+		count[a] = (uint32_t)at;
+}
+
+struct PairWork {
+	const float4* __restrict__ sp;
+	const float4* __restrict__ sn;
+	const uint2* __restrict__ pairs;
+	uint32_t npairs;
+};
+
+// One wave per cluster pair: the bit matrix of the pairs that pass
+// pair_factor (row: a patch of the first cluster) and their number.  A lane
+// keeps its patch of the second cluster; the first cluster's patches are
+// uniform.  Bound by instruction issue, about 30 a pair of patches.
+__global__ __launch_bounds__(kBlock) void k_cluster_masks(PairWork W, const uint16_t* __restrict__ quarters,
+                                                          uint64_t* __restrict__ mask, uint32_t* __restrict__ ncand)
+{
+	const uint32_t lane = threadIdx.x & 63;
+	const uint32_t p = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+	if (p >= W.npairs)
+		return;
+	const uint2 ab = W.pairs[p];
+	const uint32_t qm = (uint32_t)__builtin_amdgcn_readfirstlane((int)quarters[p]);
+	const size_t a0 = (size_t)ab.x * kCl;
+	const float4 jp = W.sp[(size_t)ab.y * kCl + lane], jn = W.sn[(size_t)ab.y * kCl + lane];
+	const f3 bp = mk3(jp.x, jp.y, jp.z), bn = mk3(jn.x, jn.y, jn.z);
+	const bool jok = __float_as_uint(jp.w) != kNoPatch;
+	const uint32_t from = ab.x == ab.y ? lane : kCl; // within a cluster: rows above the diagonal
+	uint64_t row = 0;
+	uint32_t n = 0;
+	for (uint32_t q = 0; q < 4; ++q) {
+		const uint32_t g = (qm >> (4 * q)) & 15u;
+		if (!g)
+			continue;
+		const bool in = jok && (g >> (lane >> 4) & 1u);
+		for (uint32_t i = 16 * q; i < 16 * q + 16; ++i) {
+			const float4 ip = W.sp[a0 + i], in_ = W.sn[a0 + i];
+			const bool ok = in && i < from && __float_as_uint(ip.w) != kNoPatch &&
+			                !(pair_factor(mk3(ip.x, ip.y, ip.z), mk3(in_.x, in_.y, in_.z), bp, bn) < 0.0f);
+			const uint64_t m = __ballot(ok);
+			row = lane == i ? m : row;
+			n += (uint32_t)__popcll(m);
+		}
+	}
+	if (lane == 0)
+		ncand[p] = n;
+	if (n)
+		mask[(size_t)p * kCl + lane] = row;
+}
+
+// The pairs that hold candidates, in order: their places before compaction
+// (of[], where their masks are) and the first of each cluster.
+__global__ void k_cluster_flags(const uint32_t* __restrict__ ncand, uint64_t n, uint32_t* __restrict__ flag)
+{
+	const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (p <= n)
+		flag[p] = p < n && ncand[p] ? 1u : 0u;
+}
+
+__global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, uint32_t nc,
+                                  const uint64_t* __restrict__ first, const uint2* __restrict__ pairs,
+                                  uint2* __restrict__ pairs2, uint32_t* __restrict__ of, uint64_t* __restrict__ first2)
+{
+	const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (p < n && at[p + 1] != at[p]) {
+		pairs2[at[p]] = pairs[p];
+		of[at[p]] = (uint32_t)p;
+	}
+	if (p <= nc)
+		first2[p] = at[first[p]];
+}
+
+// The occlusion tests, one wave per patch i of a cluster: its candidates in
+// the cluster's partners, 64 partners at a time, through a queue in LDS into
+// batches of 64.  A pair links when the segment between the patches hits a
+// shadow caster (VisibilityTest returns the any-hit query's hit,
+// lighter.cpp:137-147, and Int_RDGenLinks keeps the pair when it is true,
+// lighter.cpp:751-752), the lower index as its start.  A batch's segments
+// share one end, and the other ends go along the clusters' Morton order, so
+// their walks take much the same nodes (batches per cluster pair, some seven
+// patches of the first cluster in each, took 19.3 ms instead of 16.4 on a
+// city of 440,003 patches with 139 M candidates).  Bound by the walks, as the
+// AO rays are: 8.5 G segments/s there, 17.2 G/s among a room's 32,768.
+// A city's whole search, kernels: 50 ms with a uniform grid's candidate list
+// (30.1 ms of pair tests, made twice; 12.6 ms of occlusion tests on the
+// list), 28 ms so (pair tests 2.4 ms); a room's 20 -> 16 ms.
+// mask: the candidates' bits in, the links' out.  cand, linked (optional): the
+// candidates and whether each linked, in any order from *ncand on.
+struct LinkWave {
+	uint32_t row[128]; // the candidates of 64 partners, from when they are queued on the links among them
+	uint16_t queue[128];
+};
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_cluster_links(
+    View V, PairWork W, const uint64_t* __restrict__ first, const uint32_t* __restrict__ of,
+    uint64_t* __restrict__ mask, unsigned long long* ncand, uint2* __restrict__ cand, uint8_t* __restrict__ linked,
+    int depth)
+{
+	extern __shared__ __align__(16) unsigned char lds_stack[];
+	__shared__ LinkWave waves[kBlock / 64];
+	constexpr uint32_t per = kCl / (kBlock / 64); // blocks per cluster
+	const uint32_t lane = threadIdx.x & 63;
+	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+	const uint32_t a = blockIdx.x / per, i = blockIdx.x % per * (kBlock / 64) + wave;
+	const float4 A = W.sp[(size_t)a * kCl + i];
+	const uint32_t ia = __float_as_uint(A.w);
+	if (ia == kNoPatch)
+		return; // the whole wave; no block barrier below
+	LdsStack st = lds_stack_of_lane(lds_stack, depth);
+	LinkWave& L = waves[wave];
+	const uint64_t end = first[a + 1];
+	for (uint64_t p0 = first[a]; p0 < end; p0 += 64) {
+		uint64_t parts;
+		{
+			const uint64_t m = p0 + lane < end ? mask[(size_t)of[p0 + lane] * kCl + i] : 0;
+			L.row[2 * lane] = (uint32_t)m;
+			L.row[2 * lane + 1] = (uint32_t)(m >> 32);
+			parts = __ballot(m != 0);
+		}
+		if (!parts)
+			continue;
+		wave_lds_sync();
+		uint32_t qn = 0;
+		for (;;) {
+			while (qn < 64 && parts) { // partners into the queue until it holds 64 candidates
+				const uint32_t q = (uint32_t)__ffsll((unsigned long long)parts) - 1u;
+				parts &= parts - 1;
+				const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)L.row[2 * q + 1]) << 32 |
+				                   (uint32_t)__builtin_amdgcn_readfirstlane((int)L.row[2 * q]);
+				if (m >> lane & 1ull)
+					L.queue[qn + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(q << 6 | lane);
+				L.row[2 * q] = L.row[2 * q + 1] = 0u;
+				qn += (uint32_t)__popcll(m);
+			}
+			if (!qn)
+				break;
+			wave_lds_sync();
+			const uint32_t n = min(qn, 64u);
+			bool l = false;
+			if (lane < n) {
+				const uint32_t e = L.queue[lane];
+				const float4 B = W.sp[(size_t)W.pairs[p0 + (e >> 6)].y * kCl + (e & 63u)];
+				const bool up = ia < __float_as_uint(B.w);
+				const f3 P = mk3(up ? A.x : B.x, up ? A.y : B.y, up ? A.z : B.z);
+				const f3 Q = mk3(up ? B.x : A.x, up ? B.y : A.y, up ? B.z : A.z);
+				l = q_segment<true, false>(V, P, Q, nullptr, st) < 1.0f;
+			}
+			wave_lds_sync();
+			if (l) {
+				const uint32_t e = L.queue[lane];
+				atomicOr(&L.row[e >> 5], 1u << (e & 31u));
+			}
+			if (cand) {
+				unsigned long long at = 0;
+				if (lane < n) {
+					at = atomicAdd(ncand, 1ull);
+					const uint32_t e = L.queue[lane];
+					const uint32_t ib = __float_as_uint(W.sp[(size_t)W.pairs[p0 + (e >> 6)].y * kCl + (e & 63u)].w);
+					cand[at] = make_uint2(min(ia, ib), max(ia, ib));
+					linked[at] = l ? 1 : 0;
+				}
+			}
+			const uint16_t rest = L.queue[64 + lane];
+			wave_lds_sync();
+			if (lane + 64 < qn)
+				L.queue[lane] = rest;
+			wave_lds_sync();
+			qn -= n;
+		}
+		if (p0 + lane < end)
+			mask[(size_t)of[p0 + lane] * kCl + i] = (uint64_t)L.row[2 * lane + 1] << 32 | L.row[2 * lane];
+		wave_lds_sync();
+	}
+}
+
+// One wave per cluster pair: its links per patch of both clusters.
+__global__ __launch_bounds__(kBlock) void k_cluster_degrees(PairWork W, const uint32_t* __restrict__ of,
+                                                            const uint64_t* __restrict__ mask,
+                                                            uint32_t* __restrict__ deg)
+{
+	const uint32_t lane = threadIdx.x & 63;
+	const uint32_t p = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+	if (p >= W.npairs)
+		return;
+	const uint2 ab = W.pairs[p];
+	const uint64_t row = mask[(size_t)of[p] * kCl + lane];
+	if (!__any(row != 0))
+		return;
+	uint32_t col = 0;
+	for (uint32_t j = 0; j < kCl; ++j) {
+		const uint32_t c = (uint32_t)__popcll(__ballot((row >> j) & 1ull));
+		col = lane == j ? c : col;
+	}
+	if (row)
+		atomicAdd(deg + __float_as_uint(W.sp[(size_t)ab.x * kCl + lane].w), (uint32_t)__popcll(row));
+	if (col)
+		atomicAdd(deg + __float_as_uint(W.sp[(size_t)ab.y * kCl + lane].w), col);
+}
+
+// One wave per cluster pair that holds links: its links into both patches'
+// rows (any order; the row sort orders them).  fill starts at zero.
+__global__ __launch_bounds__(kBlock) void k_cluster_fill(PairWork W, const uint32_t* __restrict__ of,
+                                                         const uint64_t* __restrict__ mask,
+                                                         const uint64_t* __restrict__ rowptr,
+                                                         uint32_t* __restrict__ fill, uint32_t* __restrict__ colx)
+{
+	const uint32_t lane = threadIdx.x & 63;
+	const uint32_t p = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+	if (p >= W.npairs)
+		return;
+	const uint2 ab = W.pairs[p];
+	const uint32_t ia = __float_as_uint(W.sp[(size_t)ab.x * kCl + lane].w), ib = __float_as_uint(W.sp[(size_t)ab.y * kCl + lane].w);
+	const uint64_t row = mask[(size_t)of[p] * kCl + lane], below = (1ull << lane) - 1ull;
+	if (!__any(row != 0))
+		return;
+	uint64_t at = row ? rowptr[ia] + atomicAdd(fill + ia, (uint32_t)__popcll(row)) : 0;
+	for (uint32_t i = 0; i < kCl; ++i) {
+		const uint64_t r = __shfl(row, (int)i), o = __shfl(at, (int)i);
+		if (r >> lane & 1ull)
+			colx[o + __popcll(r & below)] = ib;
+	}
+	uint64_t col = 0;
+	for (uint32_t j = 0; j < kCl; ++j) {
+		const uint64_t c = __ballot((row >> j) & 1ull);
+		col = lane == j ? c : col;
+	}
+	at = col ? rowptr[ib] + atomicAdd(fill + ib, (uint32_t)__popcll(col)) : 0;
+	for (uint32_t j = 0; j < kCl; ++j) {
+		const uint64_t c = __shfl(col, (int)j), o = __shfl(at, (int)j);
+		if (c >> lane & 1ull)
+			colx[o + __popcll(c & below)] = ia;
+	}
 }
 
 // The occlusion test of each candidate: the pair links when the segment
@@ -1957,17 +2299,30 @@ __global__ void k_scan_blocks(const uint32_t* __restrict__ in, uint64_t n, uint6
 		block_sums[blockIdx.x] = sh[threadIdx.x];
 }
 
-__global__ void k_scan_sums(uint64_t* sums, uint32_t nb, uint64_t* total)
+// one block: each thread's run of block sums, the runs' scan, the runs again
+__global__ __launch_bounds__(kBlock) void k_scan_sums(uint64_t* sums, uint32_t nb, uint64_t* total)
 {
-	if (threadIdx.x == 0 && blockIdx.x == 0) {
-		uint64_t s = 0;
-		for (uint32_t b = 0; b < nb; ++b) {
-			uint64_t v = sums[b];
-			sums[b] = s;
-			s += v;
-		}
-		*total = s;
+	__shared__ uint64_t sh[kBlock];
+	const uint32_t per = (nb + kBlock - 1) / kBlock, b0 = min(nb, threadIdx.x * per), b1 = min(nb, b0 + per);
+	uint64_t s = 0;
+	for (uint32_t b = b0; b < b1; ++b)
+		s += sums[b];
+	sh[threadIdx.x] = s;
+	__syncthreads();
+	for (int off = 1; off < kBlock; off <<= 1) {
+		const uint64_t v = threadIdx.x >= (unsigned)off ? sh[threadIdx.x - off] : 0;
+		__syncthreads();
+		sh[threadIdx.x] += v;
+		__syncthreads();
 	}
+	uint64_t run = sh[threadIdx.x] - s;
+	for (uint32_t b = b0; b < b1; ++b) {
+		const uint64_t v = sums[b];
+		sums[b] = run;
+		run += v;
+	}
+	if (threadIdx.x == kBlock - 1)
+		*total = run;
 }
 
 __global__ void k_scan_add(uint64_t* out, uint64_t n, const uint64_t* sums)
@@ -3309,7 +3664,7 @@ static void scan_u32_to_u64(const uint32_t* d_in, uint64_t n, uint64_t* d_out, u
 	}
 	uint64_t* sums = dalloc<uint64_t>(nb + 1);
 	k_scan_blocks<<<nb, kBlock, 0, s>>>(d_in, n, d_out, sums);
-	k_scan_sums<<<1, 1, 0, s>>>(sums, nb, sums + nb);
+	k_scan_sums<<<1, kBlock, 0, s>>>(sums, nb, sums + nb);
 	k_scan_add<<<nb, kBlock, 0, s>>>(d_out, n, sums);
 	HIPCHECK(hipGetLastError());
 	HIPCHECK(hipMemcpyAsync(h_total, sums + nb, 8, hipMemcpyDeviceToHost, s));
@@ -3373,96 +3728,164 @@ void* DeviceScene::link_candidates_all(uint64_t& ncand, uint64_t* coff)
 	return cand;
 }
 
-// The same candidate set from the 27 grid cells around each patch.
-void* DeviceScene::link_candidates_grid(uint64_t& ncand, uint64_t* coff)
+// The links over clusters of patches: degrees, CSR offsets and columns (in
+// any order within a row).  Returns the entries; colx: the columns.
+uint64_t DeviceScene::links_by_clusters(uint32_t** colx)
 {
 	hipStream_t s = (hipStream_t)stream_;
 	const uint32_t N = (uint32_t)npatches;
-	ncand = 0;
-	// the longest linking distance (1 per mille margin over the float
-	// rounding of the factor); cells of half that distance (1e-4 above),
-	// searched two cells to each side: every pair within the distance is
-	// at most two cells apart per axis, and the searched box is 2.5 rather
-	// than 3 distances wide (about 40 % fewer pair tests than whole cells)
-	const double r2 = links_nmax2_ / (M_PI * (double)kSmall) * 1.001;
-	if (!(r2 > 0.0)) { // zero normals: no pair passes
-		HIPCHECK(hipMemsetAsync(coff, 0, 8 * ((size_t)N + 1), s));
-		HIPCHECK(hipStreamSynchronize(s));
-		return dalloc<uint2>(0);
-	}
-	double h = std::sqrt(r2) / 2 * 1.0001;
-	LinkGrid G;
-	G.reach = 2;
-	double na[3], cells = 0;
-	for (;;) { // sized in double: a large extent over a short distance must not overflow the counts
-		cells = 1;
-		for (int a = 0; a < 3; ++a) {
-			na[a] = std::floor(((double)links_hi_[a] - links_lo_[a]) / h) + 1;
-			cells *= na[a];
-		}
-		if (cells <= (double)(1u << 24))
-			break;
-		h *= 1.26; // wider cells keep every linking pair within reach
-	}
-	for (int a = 0; a < 3; ++a) {
-		G.lo[a] = links_lo_[a];
-		G.n[a] = (uint32_t)na[a];
-	}
-	G.inv = (float)(1.0 / h);
-	const uint32_t nc = G.n[0] * G.n[1] * G.n[2];
-	DevArray<uint32_t> cell(N), ccount(nc + 1), order(N), counts((uint64_t)N + 1);
-	DevArray<uint64_t> cstart(nc + 1);
-	HIPCHECK(hipMemsetAsync(ccount.p, 0, 4 * ((size_t)nc + 1), s));
-	k_grid_count<<<grid_for(N), kBlock, 0, s>>>(rad.pos, N, G, cell.p, ccount.p);
-	HIPCHECK(hipGetLastError());
-	if (links_mode == 0 && npatches <= kMaxAllPairsPatches) {
-		// the pairs the grid tests (both orders, each patch against the
-		// cells within reach) against the all-pairs loop's N^2 / 2: where
-		// the grid does not prune (a room within one linking distance), the
-		// loop is faster
-		std::vector<uint32_t> hist(nc);
-		HIPCHECK(hipMemcpyAsync(hist.data(), ccount.p, 4 * (size_t)nc, hipMemcpyDeviceToHost, s));
-		HIPCHECK(hipStreamSynchronize(s));
-		double tests = 0;
-		for (uint32_t z = 0; z < G.n[2]; ++z)
-			for (uint32_t y = 0; y < G.n[1]; ++y)
-				for (uint32_t x = 0; x < G.n[0]; ++x) {
-					const uint32_t c = (z * G.n[1] + y) * G.n[0] + x;
-					if (!hist[c])
-						continue;
-					double nb = 0;
-					const uint32_t q = (uint32_t)G.reach;
-					for (uint32_t zz = z > q ? z - q : 0; zz <= std::min(z + q, G.n[2] - 1); ++zz)
-						for (uint32_t yy = y > q ? y - q : 0; yy <= std::min(y + q, G.n[1] - 1); ++yy)
-							for (uint32_t xx = x > q ? x - q : 0; xx <= std::min(x + q, G.n[0] - 1); ++xx)
-								nb += hist[(zz * G.n[1] + yy) * G.n[0] + xx];
-					tests += (double)hist[c] * nb;
+	const uint32_t nc = (N + kCl - 1) / kCl, ns = (nc + kCl - 1) / kCl, Npad = nc * kCl;
+	View V = make_view(d_nodes_, d_dtri_, d_rtri_, ntri_, lo_, hi_, grid_, use_grid_ ? grid_base_ : 0, use_grid_ ? grid_fine_ : 0);
+	DevArray<float4> sp(Npad), sn(Npad);
+	{
+		// cells of a sixteenth of the longest linking distance (l^2 <= |nA| |nB|
+		// / (pi kSmall): 17.8 m for unit normals), 2^24 bins at most; sized in
+		// double, which a large extent does not overflow
+		double w = std::sqrt(links_nmax2_ / (M_PI * (double)kSmall)) / 16, cells;
+		for (int a = 0; a < 3; ++a)
+			w = std::max(w, ((double)links_hi_[a] - links_lo_[a]) * 1e-6);
+		w = std::max(w, 1e-30);
+		PatchBins G;
+		for (;; w *= 1.26) {
+			cells = 6;
+			for (int a = 0; a < 3; ++a) {
+				const double n = std::floor(((double)links_hi_[a] - links_lo_[a]) / w) + 1;
+				for (G.bits[a] = 0; std::ldexp(1.0, (int)G.bits[a]) < n; ++G.bits[a]) {
 				}
-		if (tests > 0.25 * (double)N * (double)N)
-			return link_candidates_all(ncand, coff);
+				cells *= std::ldexp(1.0, (int)G.bits[a]);
+			}
+			if (cells <= (double)(1u << 24))
+				break;
+		}
+		for (int a = 0; a < 3; ++a)
+			G.lo[a] = links_lo_[a];
+		G.inv = (float)(1.0 / w);
+		const size_t nb = (size_t)cells;
+		DevArray<uint32_t> bin(N), count(nb + 1);
+		DevArray<uint64_t> start(nb + 1);
+		HIPCHECK(hipMemsetAsync(count.p, 0, 4 * (nb + 1), s));
+		k_patch_bins<<<grid_for(N), kBlock, 0, s>>>(rad.pos, rad.nrm, N, G, bin.p, count.p);
+		HIPCHECK(hipGetLastError());
+		uint64_t total = 0;
+		scan_u32_to_u64(count.p, nb + 1, start.p, &total, s);
+		k_patch_place<<<grid_for(Npad), kBlock, 0, s>>>(rad.pos, rad.nrm, N, Npad, bin.p, start.p, count.p, sp.p, sn.p);
+		HIPCHECK(hipGetLastError());
+		HIPCHECK(hipStreamSynchronize(s)); // before bin .. start go
 	}
-	uint64_t total = 0;
-	scan_u32_to_u64(ccount.p, (uint64_t)nc + 1, cstart.p, &total, s);
-	HIPCHECK(hipMemsetAsync(ccount.p, 0, 4 * ((size_t)nc + 1), s));
-	k_grid_fill<<<grid_for(N), kBlock, 0, s>>>(N, cell.p, cstart.p, ccount.p, order.p);
-	HIPCHECK(hipMemsetAsync(counts.p + N, 0, 4, s));
-	k_pairs_grid<false><<<grid_for(N), kBlock, 0, s>>>(rad.pos, rad.nrm, N, G, cell.p, cstart.p, order.p, counts.p,
-	                                                   nullptr, nullptr);
+	DevArray<ClBox> box(nc), quart(4 * (size_t)nc), sup(ns);
+	DevArray<uint32_t> count((uint64_t)nc + 1);
+	DevArray<uint64_t> coff((uint64_t)nc + 1);
+	k_cluster_boxes<<<gridn_waves(nc), kBlock, 0, s>>>(sp.p, sn.p, nc, box.p, quart.p);
+	k_super_boxes<<<gridn_waves(ns), kBlock, 0, s>>>(box.p, nc, ns, sup.p);
+	HIPCHECK(hipMemsetAsync(count.p + nc, 0, 4, s));
+	k_cluster_pairs<false><<<gridn_waves(nc), kBlock, 0, s>>>(box.p, quart.p, nc, sup.p, ns, count.p, nullptr, nullptr, nullptr);
 	HIPCHECK(hipGetLastError());
-	scan_u32_to_u64(counts.p, (uint64_t)N + 1, coff, &ncand, s);
-	uint2* cand = dalloc<uint2>(ncand);
-	k_pairs_grid<true><<<grid_for(N), kBlock, 0, s>>>(rad.pos, rad.nrm, N, G, cell.p, cstart.p, order.p, nullptr,
-	                                                  coff, cand);
+	uint64_t npairs = 0;
+	scan_u32_to_u64(count.p, (uint64_t)nc + 1, coff.p, &npairs, s);
+	if (npairs >= (1ull << 32))
+		throw std::runtime_error("radiosity: more than 2^32 cluster pairs within linking distance");
+	DevArray<uint2> pairs(npairs);
+	DevArray<uint16_t> quarters(npairs);
+	k_cluster_pairs<true><<<gridn_waves(nc), kBlock, 0, s>>>(box.p, quart.p, nc, sup.p, ns, nullptr, coff.p, pairs.p, quarters.p);
 	HIPCHECK(hipGetLastError());
-	HIPCHECK(hipStreamSynchronize(s));
-	return cand;
+	const PairWork W{sp.p, sn.p, pairs.p, (uint32_t)npairs};
+	DevArray<uint64_t> mask(npairs * kCl);
+	DevArray<uint32_t> ncand(npairs + 1), of(npairs), deg((uint64_t)N + 1);
+	DevArray<uint2> pairs2(npairs);
+	DevArray<uint64_t> first2((uint64_t)nc + 1);
+	HIPCHECK(hipMemsetAsync(deg.p, 0, 4 * ((size_t)N + 1), s));
+	uint64_t nnz = 0, nfull = 0;
+	PairWork F{sp.p, sn.p, pairs2.p, 0}; // the pairs that hold candidates
+	if (npairs) {
+		k_cluster_masks<<<gridn_waves(npairs), kBlock, 0, s>>>(W, quarters.p, mask.p, ncand.p);
+		HIPCHECK(hipGetLastError());
+		DevArray<uint64_t> at(npairs + 1);
+		DevArray<unsigned long long> cursor(1);
+		uint2* cand = nullptr;
+		uint8_t* linked = nullptr;
+		if (count_queries) { // the candidates are kept for reference_counts_links
+			HIPCHECK(hipMemsetAsync(ncand.p + npairs, 0, 4, s));
+			scan_u32_to_u64(ncand.p, npairs + 1, at.p, &ncand_, s);
+			d_cand_ = cand = dalloc<uint2>(ncand_);
+			d_clinked_ = linked = dalloc<uint8_t>(ncand_);
+			HIPCHECK(hipMemsetAsync(cursor.p, 0, 8, s));
+		}
+		DevArray<uint32_t> flag(npairs + 1);
+		k_cluster_flags<<<grid_for(npairs + 1), kBlock, 0, s>>>(ncand.p, npairs, flag.p);
+		HIPCHECK(hipGetLastError());
+		scan_u32_to_u64(flag.p, npairs + 1, at.p, &nfull, s);
+		F.npairs = (uint32_t)nfull;
+		k_cluster_compact<<<grid_for(std::max<uint64_t>(npairs, (uint64_t)nc + 1)), kBlock, 0, s>>>(
+		    npairs, at.p, nc, coff.p, pairs.p, pairs2.p, of.p, first2.p);
+		HIPCHECK(hipGetLastError());
+		if (nfull) {
+			k_cluster_links<<<nc * (kCl / (kBlock / 64)), kBlock, march_lds_bytes(), s>>>(
+			    V, F, first2.p, of.p, mask.p, cursor.p, cand, linked, march_stack_depth());
+			HIPCHECK(hipGetLastError());
+			k_cluster_degrees<<<gridn_waves(nfull), kBlock, 0, s>>>(F, of.p, mask.p, deg.p);
+			HIPCHECK(hipGetLastError());
+		}
+		HIPCHECK(hipStreamSynchronize(s)); // before at .. flag go
+	}
+	scan_u32_to_u64(deg.p, (uint64_t)N + 1, rad.rowptr64, &nnz, s);
+	*colx = dalloc<uint32_t>(nnz);
+	if (nnz) {
+		HIPCHECK(hipMemsetAsync(deg.p, 0, 4 * ((size_t)N + 1), s)); // the rows' cursors
+		k_cluster_fill<<<gridn_waves(nfull), kBlock, 0, s>>>(F, of.p, mask.p, rad.rowptr64, deg.p, *colx);
+		HIPCHECK(hipGetLastError());
+	}
+	HIPCHECK(hipStreamSynchronize(s)); // before the arrays here go
+	return nnz;
+}
+
+// The same from all pairs, as the reference enumerates them: candidates, an
+// occlusion test of each, links per row below the diagonal (atomics from the
+// other end) and above it (the row's own candidates).
+uint64_t DeviceScene::links_by_all_pairs(uint32_t** colx)
+{
+	hipStream_t s = (hipStream_t)stream_;
+	const uint32_t N = (uint32_t)npatches;
+	View V = make_view(d_nodes_, d_dtri_, d_rtri_, ntri_, lo_, hi_, grid_, use_grid_ ? grid_base_ : 0, use_grid_ ? grid_fine_ : 0);
+	DevArray<uint64_t> coff((uint64_t)N + 1); // first candidate of each row
+	uint64_t ncand = 0;
+	uint2* cand = (uint2*)link_candidates_all(ncand, coff.p);
+	d_cand_ = cand;
+	uint8_t* linked = dalloc<uint8_t>(ncand);
+	d_clinked_ = linked;
+	DevArray<uint32_t> lower((uint64_t)N + 1), upper((uint64_t)N + 1), cnt((uint64_t)N + 1);
+	HIPCHECK(hipMemsetAsync(lower.p, 0, 4 * ((size_t)N + 1), s));
+	HIPCHECK(hipMemsetAsync(cnt.p, 0, 4 * ((size_t)N + 1), s));
+	if (ncand) {
+		k_link_test<<<grid_for(ncand), kBlock, march_lds_bytes(), s>>>(V, rad.pos, cand, ncand, linked, lower.p,
+		                                                               march_stack_depth());
+		HIPCHECK(hipGetLastError());
+	}
+	k_link_upper<<<gridn_waves(N), kBlock, 0, s>>>(N, coff.p, cand, linked, upper.p, nullptr, nullptr, nullptr);
+	k_row_sum<<<grid_for(N), kBlock, 0, s>>>(N, upper.p, lower.p, cnt.p);
+	HIPCHECK(hipGetLastError());
+	uint64_t nnz = 0;
+	scan_u32_to_u64(cnt.p, (uint64_t)N + 1, rad.rowptr64, &nnz, s);
+	*colx = dalloc<uint32_t>(nnz);
+	if (nnz) {
+		k_link_upper<<<gridn_waves(N), kBlock, 0, s>>>(N, coff.p, cand, linked, nullptr, rad.rowptr64, lower.p, *colx);
+		HIPCHECK(hipMemsetAsync(upper.p, 0, 4 * ((size_t)N + 1), s)); // the lower parts' fill counters
+		k_link_lower<<<grid_for(ncand), kBlock, 0, s>>>(cand, linked, ncand, rad.rowptr64, upper.p, *colx);
+		HIPCHECK(hipGetLastError());
+	}
+	HIPCHECK(hipStreamSynchronize(s)); // before the arrays here go
+	if (count_queries) { // the candidates are kept for reference_counts_links
+		ncand_ = ncand;
+	} else {
+		dfree(d_cand_);
+		dfree(d_clinked_);
+	}
+	return nnz;
 }
 
 size_t DeviceScene::rad_links()
 {
 	hipStream_t s = (hipStream_t)stream_;
 	const uint32_t N = (uint32_t)npatches;
-	View V = make_view(d_nodes_, d_dtri_, d_rtri_, ntri_, lo_, hi_, grid_, use_grid_ ? grid_base_ : 0, use_grid_ ? grid_fine_ : 0);
 	dfree(rad.rowptr);
 	dfree(rad.rowptr64);
 	dfree(rad.col);
@@ -3473,68 +3896,36 @@ size_t DeviceScene::rad_links()
 	rad.nnz = 0;
 	rad.rowptr64 = dalloc<uint64_t>((uint64_t)N + 1);
 	EventTimer tm(s);
-	uint64_t ncand = 0;
-	uint2* cand = nullptr;
-	DevArray<uint64_t> coff((uint64_t)N + 1); // first candidate of each row
-	if (N > 1) {
-		cand = (uint2*)((links_mode == 1 || !links_finite_) ? link_candidates_all(ncand, coff.p)
-		                                                    : link_candidates_grid(ncand, coff.p));
-	} else {
-		HIPCHECK(hipMemsetAsync(coff.p, 0, 8 * ((size_t)N + 1), s));
-	}
-	// occlusion test of every candidate; links per row below the diagonal
-	// (atomics from the other end) and above it (the row's own candidates)
-	DevArray<uint32_t> lower((uint64_t)N + 1), upper((uint64_t)N + 1), cnt((uint64_t)N + 1);
-	HIPCHECK(hipMemsetAsync(lower.p, 0, 4 * ((size_t)N + 1), s));
-	HIPCHECK(hipMemsetAsync(cnt.p, 0, 4 * ((size_t)N + 1), s));
-	uint8_t* linked = dalloc<uint8_t>(ncand);
-	if (ncand) {
-		k_link_test<<<grid_for(ncand), kBlock, march_lds_bytes(), s>>>(V, rad.pos, cand, ncand, linked, lower.p,
-		                                                               march_stack_depth());
-		HIPCHECK(hipGetLastError());
-	}
-	if (N) {
-		k_link_upper<<<gridn_waves(N), kBlock, 0, s>>>(N, coff.p, cand, linked, upper.p, nullptr, nullptr, nullptr);
-		k_row_sum<<<grid_for(N), kBlock, 0, s>>>(N, upper.p, lower.p, cnt.p);
-		HIPCHECK(hipGetLastError());
-	}
+	uint32_t* colx = nullptr;
+	struct Free {
+		uint32_t*& p;
+		~Free() { dfree(p); }
+	} fr{colx};
 	// symmetric CSR, columns ascending within a row; 32-bit row offsets too
 	// while they fit (the solver forms take those)
 	uint64_t nnz = 0;
-	scan_u32_to_u64(cnt.p, (uint64_t)N + 1, rad.rowptr64, &nnz, s);
+	if (N > 1) {
+		nnz = links_mode == 1 || !links_finite_ ? links_by_all_pairs(&colx) : links_by_clusters(&colx);
+	} else {
+		HIPCHECK(hipMemsetAsync(rad.rowptr64, 0, 8 * ((size_t)N + 1), s));
+	}
 	if (nnz < (1ull << 32)) {
 		rad.rowptr = dalloc<uint32_t>((uint64_t)N + 1);
 		k_u64_to_u32<<<grid_for((uint64_t)N + 1), kBlock, 0, s>>>(rad.rowptr64, (uint64_t)N + 1, rad.rowptr);
 		HIPCHECK(hipGetLastError());
 	}
-	HIPCHECK(hipStreamSynchronize(s));
 	rad.nnz = nnz;
 	rad.col = dalloc<uint32_t>(nnz);
 	rad.val = dalloc<float>(nnz);
 	if (nnz) {
-		DevArray<uint32_t> colx(nnz);
-		k_link_upper<<<gridn_waves(N), kBlock, 0, s>>>(N, coff.p, cand, linked, nullptr, rad.rowptr64, lower.p,
-		                                                colx.p);
-		HIPCHECK(hipMemsetAsync(upper.p, 0, 4 * ((size_t)N + 1), s)); // the lower parts' fill counters
-		k_link_lower<<<grid_for(ncand), kBlock, 0, s>>>(cand, linked, ncand, rad.rowptr64, upper.p, colx.p);
-		HIPCHECK(hipGetLastError());
 		int bits = 1;
 		while (bits < 32 && (1ull << bits) < N)
 			++bits;
-		sort_row_columns(colx.p, rad.col, nnz, N, rad.rowptr64, bits, s);
+		sort_row_columns(colx, rad.col, nnz, N, rad.rowptr64, bits, s);
 		k_link_factors<<<gridn_waves(N), kBlock, 0, s>>>(N, rad.rowptr64, rad.col, rad.pos, rad.nrm, rad.val);
 		HIPCHECK(hipGetLastError());
-		HIPCHECK(hipStreamSynchronize(s)); // before colx goes
 	}
-	HIPCHECK(hipStreamSynchronize(s));
-	if (count_queries) { // kept for reference_counts_links
-		d_cand_ = (void*)cand;
-		d_clinked_ = (void*)linked;
-		ncand_ = ncand;
-	} else {
-		dfree(cand);
-		dfree(linked);
-	}
+	HIPCHECK(hipStreamSynchronize(s)); // before colx goes
 	times.links_ms = tm.stop();
 	nlinks_ = nnz / 2;
 	return nlinks_;
