@@ -1955,23 +1955,98 @@ __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, u
 // share one end, and the other ends go along the clusters' Morton order, so
 // their walks take much the same nodes (batches per cluster pair, some seven
 // patches of the first cluster in each, took 19.3 ms instead of 16.4 on a
-// city of 440,003 patches with 139 M candidates).  Bound by the walks, as the
-// AO rays are: 8.5 G segments/s there, 17.2 G/s among a room's 32,768.
-// A city's whole search, kernels: 50 ms with a uniform grid's candidate list
-// (30.1 ms of pair tests, made twice; 12.6 ms of occlusion tests on the
-// list), 28 ms so (pair tests 2.4 ms); a room's 20 -> 16 ms.
+// city of 440,003 patches with 139 M candidates).  Bound by the walks' issue
+// and node fetches.  A city's whole search, kernels: 50 ms with a uniform
+// grid's candidate list (30.1 ms of pair tests, made twice; 12.6 ms of
+// occlusion tests on the list), 26 ms so (pair tests 2.4 ms); a room's 20 ->
+// 12 ms.
 // mask: the candidates' bits in, the links' out.  cand, linked (optional): the
 // candidates and whether each linked, in any order from *ncand on.
+//
+// The walk is one for the wave: all 64 segments go to a node that any of
+// them meets, so a node's and a triangle's data are the same on every lane,
+// nothing is sorted per lane and the stack is one list of references.  A
+// segment that would have passed a node by takes its children's tests too;
+// whether it is hit by some triangle does not depend on that.  The nodes and
+// triangles come through scalar loads.  Against a walk per lane: a room's
+// 12.7 -> 8.8 ms (25 G segments/s), a city's 16.4 -> 14.5 ms.
+typedef __attribute__((address_space(4))) const v4f const_v4f; // read-only for the kernel: scalar loads
+typedef int32_t v4i __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(4))) const v4i const_v4i;
+
+__device__ __forceinline__ uint64_t wave_occluded(const View& V, f3 A, f3 P, f3 Q, bool live, uint32_t* stack)
+{
+	uint64_t alive = __ballot(live), hit = 0;
+	if (!V.has_tris || !alive)
+		return 0;
+	const Seg s = make_seg(P, Q);
+	// segments of at most kGridReach from A start at its cell
+	const f3 d = Q - P;
+	int32_t ref = __any(live && !(dot(d, d) <= kGridReach * kGridReach)) ? 0 : entry_node(V, A);
+	ref = __builtin_amdgcn_readfirstlane(ref);
+	uint32_t sp = 0;
+	for (;;) {
+		if (ref >= 0) {
+			const_v4f* q = (const_v4f*)(uintptr_t)(V.nodes + ref);
+			const v4f lx = q[0], ly = q[1], lz = q[2], hx = q[3], hy = q[4], hz = q[5];
+			const v4i c = *(const_v4i*)(uintptr_t)(V.nodes[ref].child);
+			const float t[4] = {slab(s, lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, 1.0f),
+			                    slab(s, lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, 1.0f),
+			                    slab(s, lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, 1.0f),
+			                    slab(s, lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, 1.0f)};
+			int32_t go = 0;
+			uint64_t most = 0;
+			bool any = false;
+#pragma unroll
+			for (int k = 0; k < 4; ++k) {
+				const uint64_t m = __ballot(t[k] != INFINITY) & alive;
+				if (!m)
+					continue;
+				// the child that most segments meet next, the others later
+				const bool first = !any || __popcll(m) > __popcll(most);
+				if (any)
+					stack[sp++] = (uint32_t)(first ? go : c[k]);
+				if (first) {
+					go = c[k];
+					most = m;
+				}
+				any = true;
+			}
+			if (any) {
+				ref = __builtin_amdgcn_readfirstlane(go);
+				continue;
+			}
+		} else {
+			const uint32_t f = leaf_first(ref), c = leaf_count(ref);
+			for (uint32_t i = 0; i < c; ++i) {
+				const_v4f* q = (const_v4f*)(uintptr_t)(V.rtri + f + i);
+				const v4f q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+				const RayTri T{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+				const float r = seg_tri_pre(s.o, s.dir, T);
+				const uint64_t h = __ballot(r < 1.0f) & alive;
+				hit |= h;
+				alive &= ~h;
+			}
+			if (!alive)
+				break;
+		}
+		if (sp == 0)
+			break;
+		wave_lds_sync();
+		ref = __builtin_amdgcn_readfirstlane((int)stack[--sp]);
+	}
+	return hit;
+}
+
 struct LinkWave {
+	uint32_t stack[kStackSize];
 	uint32_t row[128]; // the candidates of 64 partners, from when they are queued on the links among them
 	uint16_t queue[128];
 };
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_cluster_links(
+__global__ __launch_bounds__(kBlock) void k_cluster_links(
     View V, PairWork W, const uint64_t* __restrict__ first, const uint32_t* __restrict__ of,
-    uint64_t* __restrict__ mask, unsigned long long* ncand, uint2* __restrict__ cand, uint8_t* __restrict__ linked,
-    int depth)
+    uint64_t* __restrict__ mask, unsigned long long* ncand, uint2* __restrict__ cand, uint8_t* __restrict__ linked)
 {
-	extern __shared__ __align__(16) unsigned char lds_stack[];
 	__shared__ LinkWave waves[kBlock / 64];
 	constexpr uint32_t per = kCl / (kBlock / 64); // blocks per cluster
 	const uint32_t lane = threadIdx.x & 63;
@@ -1981,7 +2056,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) 
 	const uint32_t ia = __float_as_uint(A.w);
 	if (ia == kNoPatch)
 		return; // the whole wave; no block barrier below
-	LdsStack st = lds_stack_of_lane(lds_stack, depth);
 	LinkWave& L = waves[wave];
 	const uint64_t end = first[a + 1];
 	for (uint64_t p0 = first[a]; p0 < end; p0 += 64) {
@@ -2011,15 +2085,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) 
 				break;
 			wave_lds_sync();
 			const uint32_t n = min(qn, 64u);
-			bool l = false;
-			if (lane < n) {
-				const uint32_t e = L.queue[lane];
-				const float4 B = W.sp[(size_t)W.pairs[p0 + (e >> 6)].y * kCl + (e & 63u)];
-				const bool up = ia < __float_as_uint(B.w);
-				const f3 P = mk3(up ? A.x : B.x, up ? A.y : B.y, up ? A.z : B.z);
-				const f3 Q = mk3(up ? B.x : A.x, up ? B.y : A.y, up ? B.z : A.z);
-				l = q_segment<true, false>(V, P, Q, nullptr, st) < 1.0f;
-			}
+			const uint32_t e0 = L.queue[min(lane, n - 1)];
+			const float4 B = W.sp[(size_t)W.pairs[p0 + (e0 >> 6)].y * kCl + (e0 & 63u)];
+			const bool up = ia < __float_as_uint(B.w);
+			const f3 P = mk3(up ? A.x : B.x, up ? A.y : B.y, up ? A.z : B.z);
+			const f3 Q = mk3(up ? B.x : A.x, up ? B.y : A.y, up ? B.z : A.z);
+			const bool l = wave_occluded(V, mk3(A.x, A.y, A.z), P, Q, lane < n, L.stack) >> lane & 1ull;
 			wave_lds_sync();
 			if (l) {
 				const uint32_t e = L.queue[lane];
@@ -3819,8 +3890,8 @@ uint64_t DeviceScene::links_by_clusters(uint32_t** colx)
 		    npairs, at.p, nc, coff.p, pairs.p, pairs2.p, of.p, first2.p);
 		HIPCHECK(hipGetLastError());
 		if (nfull) {
-			k_cluster_links<<<nc * (kCl / (kBlock / 64)), kBlock, march_lds_bytes(), s>>>(
-			    V, F, first2.p, of.p, mask.p, cursor.p, cand, linked, march_stack_depth());
+			k_cluster_links<<<nc * (kCl / (kBlock / 64)), kBlock, 0, s>>>(
+			    V, F, first2.p, of.p, mask.p, cursor.p, cand, linked);
 			HIPCHECK(hipGetLastError());
 			k_cluster_degrees<<<gridn_waves(nfull), kBlock, 0, s>>>(F, of.p, mask.p, deg.p);
 			HIPCHECK(hipGetLastError());
