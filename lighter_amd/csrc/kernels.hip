@@ -1052,6 +1052,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 constexpr float kFaceNear = 0.25f; // steps shorter than this try the face interval
 constexpr int kGatherQueue = 256; // node references in flight per wave (a power of two)
 
+__device__ __forceinline__ float lane_value(float v, int lane)
+{
+	return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
 // minimum over the 64 lanes (all active), the same on every lane
 __device__ __forceinline__ float wave_min(float v)
 {
@@ -1161,11 +1166,6 @@ __device__ __forceinline__ float face_slack(f3 p, const DistTri& T)
 	const float v0 = fmaxf(t0p - T.t0min, T.t2max - t2p), v1 = fmaxf(t1p - T.t1min, T.t0max - t0p);
 	const float v2 = fmaxf(t2p - T.t2min, T.t1max - t1p);
 	return fminf(fminf(fminf(v0, v1), v2), -fmaxf(fmaxf(ptd0, ptd1), ptd2));
-}
-
-__device__ __forceinline__ float lane_value(float v, int lane)
-{
-	return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 // march_step's steps up to t = face, the distance that of the plane (n, d);
@@ -1359,11 +1359,127 @@ __device__ __forceinline__ float wave_uniform(float x)
 	return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
 }
 
+// ---------------------------------------------------------------------------
+// One walk for a wave's 64 segments: the wave goes to every node that any of
+// them meets, so a node's and a triangle's data are the same on every lane
+// (scalar loads), nothing is sorted per lane and the stack is one list of
+// references in LDS.  A segment that would have passed a node by takes its
+// children's tests too; whether it is hit at all does not depend on that.
+// (For the rays of ambient occlusion, which part in all directions, it lost:
+// 64 rays a texel on a terrain 5.26 ms against 3.95 with a walk per lane.)
+// ---------------------------------------------------------------------------
+typedef __attribute__((address_space(4))) const v4f const_v4f; // read-only for the kernel: scalar loads
+typedef int32_t v4i __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(4))) const v4i const_v4i;
+
+
+// The children of node ref that live lanes meet within tlim: the one that
+// most meet is returned, the others go onto the stack; kNoNode for none.
+constexpr int32_t kNoNode = INT32_MIN;
+__device__ __forceinline__ int32_t wave_children(const View& V, int32_t ref, const Seg& s, float tlim, uint64_t alive,
+                                                 uint32_t* stack, uint32_t& sp)
+{
+	const_v4f* q = (const_v4f*)(uintptr_t)(V.nodes + ref);
+	const v4f lx = q[0], ly = q[1], lz = q[2], hx = q[3], hy = q[4], hz = q[5];
+	const v4i c = *(const_v4i*)(uintptr_t)(V.nodes[ref].child);
+	const float t[4] = {slab(s, lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, tlim), slab(s, lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, tlim),
+	                    slab(s, lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, tlim), slab(s, lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, tlim)};
+	int32_t go = kNoNode;
+	uint64_t most = 0;
+#pragma unroll
+	for (int k = 0; k < 4; ++k) {
+		const uint64_t m = __ballot(t[k] != INFINITY) & alive;
+		if (!m)
+			continue;
+		const bool first = !most || __popcll(m) > __popcll(most);
+		if (most)
+			stack[sp++] = (uint32_t)(first ? go : c[k]);
+		if (first) {
+			go = c[k];
+			most = m;
+		}
+	}
+	return __builtin_amdgcn_readfirstlane(go);
+}
+
+__device__ __forceinline__ float wave_leaf_tri(const View& V, uint32_t f, const Seg& s)
+{
+	const_v4f* q = (const_v4f*)(uintptr_t)(V.rtri + f);
+	const v4f q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+	const RayTri T{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+	return seg_tri_pre(s.o, s.dir, T);
+}
+
+// lanes whose segment P -> Q hits a triangle with r < 1; A: an end that all
+// live segments share
+__device__ __forceinline__ uint64_t wave_occluded(const View& V, f3 A, f3 P, f3 Q, bool live, uint32_t* stack)
+{
+	uint64_t alive = __ballot(live), hit = 0;
+	if (!V.has_tris || !alive)
+		return 0;
+	const Seg s = make_seg(P, Q);
+	// segments of at most kGridReach from A start at its cell
+	const f3 d = Q - P;
+	int32_t ref = __any(live && !(dot(d, d) <= kGridReach * kGridReach)) ? 0 : entry_node(V, A);
+	ref = __builtin_amdgcn_readfirstlane(ref);
+	uint32_t sp = 0;
+	for (;;) {
+		if (ref >= 0) {
+			ref = wave_children(V, ref, s, 1.0f, alive, stack, sp);
+			if (ref != kNoNode)
+				continue;
+		} else {
+			const uint32_t f = leaf_first(ref), c = leaf_count(ref);
+			for (uint32_t i = 0; i < c; ++i) {
+				const uint64_t h = __ballot(wave_leaf_tri(V, f + i, s) < 1.0f) & alive;
+				hit |= h;
+				alive &= ~h;
+			}
+			if (!alive)
+				break;
+		}
+		if (sp == 0)
+			break;
+		wave_lds_sync();
+		ref = __builtin_amdgcn_readfirstlane((int)stack[--sp]);
+	}
+	return hit;
+}
+
 struct AOParams {
 	int n;
 	float distance, multiplier, falloff, effect;
 	float color[3];
 };
+
+// sum plus the terms of the lanes in `of`, in ray order; only the rays that
+// hit something: the others would add zero to a sum that is not negative.
+__device__ __forceinline__ float add_terms(float sum, float term, uint64_t of)
+{
+	for (uint64_t h = __ballot(term != 0.0f) & of; h; h &= h - 1)
+		sum += lane_value(term, __ffsll((unsigned long long)h) - 1);
+	return sum;
+}
+
+// the texel's factor from the sum of its rays' terms, and its colour
+__device__ __forceinline__ void ao_blend(uint32_t s, float ao, const AOParams& P, float* __restrict__ lm,
+                                         float* __restrict__ fac_out)
+{
+	ao /= P.n;
+	ao = tmin(ao * P.multiplier, 1.0f);
+	if (P.falloff)
+		ao = pow_r(ao, P.falloff);
+	if (fac_out)
+		fac_out[s] = ao;
+	f3 out = ld3(lm + 3 * s);
+	f3 col = mk3(P.color[0], P.color[1], P.color[2]);
+	if (P.effect >= 0) {
+		out = out * (1 - ao * (1 - P.effect)) + col * ao;
+	} else {
+		out = lerp3(out, lerp3(col, col * out, -P.effect), ao);
+	}
+	st3(lm + 3 * s, out);
+}
 
 // One wave per texel, one lane per ray (rays beyond 64 in further rounds of
 // the wave): the rays of a texel start together and stay coherent, and a
@@ -1410,31 +1526,52 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 			float2 sd = side[i];
 			f3 d = spiral_dir(SN, sd.x, sd.y, (float)ca, (float)sa) * P.distance;
 			asm volatile("" ::"v"(touch));
-			float hit = q_segment<false, COUNT>(V, origin, origin + d, cnt, st, start);
+			const float hit = q_segment<false, COUNT>(V, origin, origin + d, cnt, st, start);
 			if (hit < 1.0f)
 				term = 1.0f - hit; // a miss adds nothing (ao + 0 = ao)
 		}
-		// every lane adds the 64 terms in ray order (the same sum on every lane)
-		const int m = P.n - i0 < 64 ? P.n - i0 : 64;
-		for (int k = 0; k < m; ++k)
-			ao += __shfl(term, k);
+		ao = add_terms(ao, term, ~0ull);
 	}
 	if (lane != 0)
 		return;
-	ao /= P.n;
-	ao = tmin(ao * P.multiplier, 1.0f);
-	if (P.falloff)
-		ao = pow_r(ao, P.falloff);
-	if (fac_out)
-		fac_out[s] = ao;
-	f3 out = ld3(lm + 3 * s);
-	f3 col = mk3(P.color[0], P.color[1], P.color[2]);
-	if (P.effect >= 0) {
-		out = out * (1 - ao * (1 - P.effect)) + col * ao;
-	} else {
-		out = lerp3(out, lerp3(col, col * out, -P.effect), ao);
+	ao_blend(s, ao, P, lm, fac_out);
+}
+
+// The same for at most 32 rays: T = 64 / n texels per wave, lane q n + i the
+// i-th ray of its q-th texel.  Bound by the walks' node fetches as k_ao is;
+// a wave per texel left 47 lanes idle at 17 rays (a city's 700,001 texels
+// 1.97 ms; packed 0.90).  Above 32 rays no second texel fits.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_ao_packed(
+    View V, const float* __restrict__ pos, const float* __restrict__ nrm, const float* __restrict__ randoff,
+    const float2* __restrict__ side, AOParams P, uint32_t s0, uint32_t S, float* __restrict__ lm, int depth,
+    float* __restrict__ fac_out)
+{
+	extern __shared__ __align__(16) unsigned char lds_stack[];
+	LdsStack st = lds_stack_of_lane(lds_stack, depth);
+	const uint32_t lane = threadIdx.x & 63, n = (uint32_t)P.n, T = 64 / n;
+	const uint32_t q = lane / n, i = lane - q * n;
+	const uint32_t s = s0 + (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * T + q;
+	const bool in = q < T && s < S;
+	float term = 0.0f;
+	if (in) {
+		const f3 SN = ld3(nrm + 3 * (size_t)s), origin = ld3(pos + 3 * (size_t)s) + SN * (kSmall * 2);
+		const float angle = (i + randoff[s]) * kGoldenAngle;
+		double sa, ca;
+		sincos((double)angle, &sa, &ca);
+		const float2 sd = side[i];
+		const f3 d = spiral_dir(SN, sd.x, sd.y, (float)ca, (float)sa) * P.distance;
+		const int32_t start = P.distance <= kGridReach ? entry_node(V, origin) : 0;
+		const float hit = q_segment<false, false>(V, origin, origin + d, nullptr, st, start);
+		if (hit < 1.0f)
+			term = 1.0f - hit;
 	}
-	st3(lm + 3 * s, out);
+	float ao = 0.0f;
+	for (uint32_t t = 0; t < T; ++t) {
+		const float a = add_terms(0.0f, term, ((n < 64 ? 1ull << n : 0ull) - 1ull) << (t * n));
+		ao = q == t ? a : ao;
+	}
+	if (in && i == 0)
+		ao_blend(s, ao, P, lm, fac_out);
 }
 
 // Closest hit of DistanceTestBBT (lighter.cpp:254-289) on the binary tree
@@ -1962,82 +2099,8 @@ __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, u
 // 12 ms.
 // mask: the candidates' bits in, the links' out.  cand, linked (optional): the
 // candidates and whether each linked, in any order from *ncand on.
-//
-// The walk is one for the wave: all 64 segments go to a node that any of
-// them meets, so a node's and a triangle's data are the same on every lane,
-// nothing is sorted per lane and the stack is one list of references.  A
-// segment that would have passed a node by takes its children's tests too;
-// whether it is hit by some triangle does not depend on that.  The nodes and
-// triangles come through scalar loads.  Against a walk per lane: a room's
+// The walk is one for the wave (wave_occluded).  Against a walk per lane: a room's
 // 12.7 -> 8.8 ms (25 G segments/s), a city's 16.4 -> 14.5 ms.
-typedef __attribute__((address_space(4))) const v4f const_v4f; // read-only for the kernel: scalar loads
-typedef int32_t v4i __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(4))) const v4i const_v4i;
-
-__device__ __forceinline__ uint64_t wave_occluded(const View& V, f3 A, f3 P, f3 Q, bool live, uint32_t* stack)
-{
-	uint64_t alive = __ballot(live), hit = 0;
-	if (!V.has_tris || !alive)
-		return 0;
-	const Seg s = make_seg(P, Q);
-	// segments of at most kGridReach from A start at its cell
-	const f3 d = Q - P;
-	int32_t ref = __any(live && !(dot(d, d) <= kGridReach * kGridReach)) ? 0 : entry_node(V, A);
-	ref = __builtin_amdgcn_readfirstlane(ref);
-	uint32_t sp = 0;
-	for (;;) {
-		if (ref >= 0) {
-			const_v4f* q = (const_v4f*)(uintptr_t)(V.nodes + ref);
-			const v4f lx = q[0], ly = q[1], lz = q[2], hx = q[3], hy = q[4], hz = q[5];
-			const v4i c = *(const_v4i*)(uintptr_t)(V.nodes[ref].child);
-			const float t[4] = {slab(s, lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, 1.0f),
-			                    slab(s, lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, 1.0f),
-			                    slab(s, lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, 1.0f),
-			                    slab(s, lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, 1.0f)};
-			int32_t go = 0;
-			uint64_t most = 0;
-			bool any = false;
-#pragma unroll
-			for (int k = 0; k < 4; ++k) {
-				const uint64_t m = __ballot(t[k] != INFINITY) & alive;
-				if (!m)
-					continue;
-				// the child that most segments meet next, the others later
-				const bool first = !any || __popcll(m) > __popcll(most);
-				if (any)
-					stack[sp++] = (uint32_t)(first ? go : c[k]);
-				if (first) {
-					go = c[k];
-					most = m;
-				}
-				any = true;
-			}
-			if (any) {
-				ref = __builtin_amdgcn_readfirstlane(go);
-				continue;
-			}
-		} else {
-			const uint32_t f = leaf_first(ref), c = leaf_count(ref);
-			for (uint32_t i = 0; i < c; ++i) {
-				const_v4f* q = (const_v4f*)(uintptr_t)(V.rtri + f + i);
-				const v4f q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
-				const RayTri T{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
-				const float r = seg_tri_pre(s.o, s.dir, T);
-				const uint64_t h = __ballot(r < 1.0f) & alive;
-				hit |= h;
-				alive &= ~h;
-			}
-			if (!alive)
-				break;
-		}
-		if (sp == 0)
-			break;
-		wave_lds_sync();
-		ref = __builtin_amdgcn_readfirstlane((int)stack[--sp]);
-	}
-	return hit;
-}
-
 struct LinkWave {
 	uint32_t stack[kStackSize];
 	uint32_t row[128]; // the candidates of 64 partners, from when they are queued on the links among them
@@ -3625,7 +3688,11 @@ void DeviceScene::ambient_occlusion(const float* randoff, int num_samples, float
 	for (size_t b = 0; b < nsamples_; b += chunk) {
 		const size_t e = std::min(nsamples_, b + chunk);
 		const unsigned ao_grid = (unsigned)((e - b + kBlock / 64 - 1) / (kBlock / 64)); // a wave per texel
-		if (count_queries)
+		if (!count_queries && num_samples <= 32) {
+			const size_t per = (size_t)(kBlock / 64) * (64 / num_samples); // texels per block
+			k_ao_packed<<<(unsigned)((e - b + per - 1) / per), kBlock, march_lds_bytes(), s>>>(
+			    V, d_pos_, d_nrm_, d_ro, d_side, P, (uint32_t)b, (uint32_t)e, d_lm_, march_stack_depth(), fac_out);
+		} else if (count_queries)
 			k_ao<true><<<ao_grid, kBlock, march_lds_bytes(), s>>>(V, d_pos_, d_nrm_, d_ro, d_side, P, (uint32_t)b,
 			                                                      (uint32_t)e, d_lm_, d_counters_,
 			                                                      march_stack_depth(), fac_out);
