@@ -239,6 +239,9 @@ private:
 	uint32_t* d_skey_ = nullptr; // 30-bit Morton code of each sample position (march ordering)
 	float* d_nrm_ = nullptr;
 	float* d_lm_ = nullptr;
+	float* d_ao_ = nullptr; // AO: rotation offsets, and the rays' side angles
+	void* d_side_ = nullptr;
+	size_t samples_cap_ = 0, ao_cap_ = 0, side_cap_ = 0;
 	void* d_cand_ = nullptr;    // candidate pairs (uint2) of the last link search, kept in counting mode
 	void* d_clinked_ = nullptr; // and whether each one linked (uint8)
 	uint64_t ncand_ = 0;

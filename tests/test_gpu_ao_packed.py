@@ -41,3 +41,28 @@ def test_packed_texels_match_wave_per_texel(lib, rays, texels):
     dev.close()
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
     assert texels < 1000 or np.any(out[0] != lm0)
+
+
+def test_sample_sets_of_changing_size(lib):
+    """One device given sample sets that grow and shrink, against a
+    new device for each."""
+    rng = np.random.default_rng(3)
+    tris = _soup(rng, 300)
+    dev = Device(lib, tris)
+    col = np.ones(3, np.float32)
+    for n in (2000, 1, 499, 2001, 700, 64, 0, 65):
+        pos = rng.uniform(-4, 4, (n, 3)).astype(np.float32)
+        nrm = rng.normal(size=(n, 3)).astype(np.float32)
+        ro = rng.uniform(0, 1, n).astype(np.float32)
+        one = Device(lib, tris)
+        out = []
+        for d in (dev, one):
+            _lib.check(lib.lgx_SetSamples(d.h, P(pos), P(nrm), n, None), lib)
+            _lib.check(lib.lgx_AmbientOcclusion(d.h, P(ro), 24, 2.0, 1.0, 1.0, 0.0, P(col)), lib)
+            got = np.zeros((n, 3), np.float32)
+            if n:
+                _lib.check(lib.lgx_ReadLightmap(d.h, P(got)), lib)
+            out.append(got)
+        one.close()
+        assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32)), n
+    dev.close()
