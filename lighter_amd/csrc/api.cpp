@@ -828,7 +828,7 @@ int lgx_SetLinkSearch(lgx_Device* d, int mode)
 {
 	return guarded([&] {
 		if (mode < 0 || mode > 2)
-			throw std::runtime_error("lgx_SetLinkSearch: mode 0 (automatic), 1 (all pairs) or 2 (grid)");
+			throw std::runtime_error("lgx_SetLinkSearch: mode 0 (automatic), 1 (all pairs) or 2 (clusters)");
 		d->dev.links_mode = mode;
 	});
 }

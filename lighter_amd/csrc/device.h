@@ -3,6 +3,8 @@
 // pipeline and by the lgx_* entry points.
 #pragma once
 
+#include <map>
+#include <mutex>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -11,6 +13,8 @@
 #include <vector>
 
 namespace lgx {
+
+class SpareBlocks;
 
 // Light as stored after ltr_LightAdd (direction normalised), as the kernels
 // read it.
@@ -45,7 +49,7 @@ constexpr size_t kMaxAllPairsPatches = 524288;
 // in -> out, nnz entries, rows given by rowptr (nrows + 1 entries, device),
 // column values below 2^bits.
 void sort_row_columns(const uint32_t* in, uint32_t* out, uint64_t nnz, uint32_t nrows, const uint64_t* rowptr,
-                      int bits, void* stream);
+                      int bits, SpareBlocks& mem, void* stream);
 
 // Per-stage timing in milliseconds measured with HIP events on the stream
 // the kernels run on.
@@ -59,6 +63,27 @@ struct StageTimes {
 struct QueryCounters {
 	unsigned long long nodes = 0, tris = 0, steps = 0, queries = 0, marches = 0;
 	unsigned long long pretests = 0; // triangles the box pre-test culled (distance queries)
+};
+
+// Scratch blocks of one device scene, kept between its calls for the next
+// that asks for much the same size; at most 8 GiB of them, given back when an
+// allocation fails and with the scene.  All work on them is on the scene's
+// one stream (copies on the null stream wait for it), which orders a block's
+// next use after its last.
+class SpareBlocks {
+public:
+	SpareBlocks() = default;
+	SpareBlocks(const SpareBlocks&) = delete;
+	SpareBlocks& operator=(const SpareBlocks&) = delete;
+	~SpareBlocks() { release(); }
+	void* take(size_t bytes, size_t* cap);
+	void give(void* p, size_t cap);
+	void release();
+
+private:
+	std::mutex mu_;
+	std::multimap<size_t, void*> spare_; // by size
+	size_t total_ = 0;
 };
 
 class DeviceScene {
@@ -239,6 +264,8 @@ private:
 	uint32_t* d_skey_ = nullptr; // 30-bit Morton code of each sample position (march ordering)
 	float* d_nrm_ = nullptr;
 	float* d_lm_ = nullptr;
+	SpareBlocks spare_;
+	size_t col_cap_ = 0, val_cap_ = 0; // bytes of rad.col and rad.val
 	float* d_ao_ = nullptr; // AO: rotation offsets, and the rays' side angles
 	void* d_side_ = nullptr;
 	size_t samples_cap_ = 0, ao_cap_ = 0, side_cap_ = 0;
@@ -252,8 +279,8 @@ private:
 	// candidate pairs (uint2, i < j, device memory), grouped by row i;
 	// coff (N + 1, device) receives the first candidate of each row
 	void* link_candidates_all(uint64_t& ncand, uint64_t* coff);
-	uint64_t links_by_all_pairs(uint32_t** colx); // CSR entries; the unsorted columns
-	uint64_t links_by_clusters(uint32_t** colx);
+	uint64_t links_by_all_pairs(uint32_t** colx, size_t* cap); // CSR entries; the unsorted columns
+	uint64_t links_by_clusters(uint32_t** colx, size_t* cap);
 	size_t nsamples_ = 0;
 	// direct light
 	float* d_w_ = nullptr;

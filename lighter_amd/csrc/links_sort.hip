@@ -31,7 +31,7 @@ __global__ void k_rel_offsets(const uint64_t* __restrict__ rowptr, uint32_t r0, 
 }
 
 void sort_row_columns(const uint32_t* in, uint32_t* out, uint64_t nnz, uint32_t nrows, const uint64_t* rowptr,
-                      int bits, void* stream)
+                      int bits, SpareBlocks& mem, void* stream)
 {
 	hipStream_t s = (hipStream_t)stream;
 	if (nnz == 0 || nrows == 0)
@@ -42,8 +42,7 @@ void sort_row_columns(const uint32_t* in, uint32_t* out, uint64_t nnz, uint32_t 
 	constexpr uint64_t kRun = (uint64_t)1 << 31;
 	uint32_t* rel = nullptr;
 	void* tmp = nullptr;
-	size_t tmp_bytes = 0;
-	uint32_t rel_cap = 0;
+	size_t rel_cap = 0, tmp_cap = 0; // bytes
 	try {
 		for (uint32_t r0 = 0; r0 < nrows;) {
 			uint32_t r1 = r0 + 1;
@@ -53,24 +52,20 @@ void sort_row_columns(const uint32_t* in, uint32_t* out, uint64_t nnz, uint32_t 
 				++r1;
 			const uint64_t base = rp[r0];
 			const uint32_t size = (uint32_t)(rp[r1] - base), nseg = r1 - r0;
-			if (nseg + 1 > rel_cap) {
-				if (rel)
-					SORTCHECK(hipFree(rel));
+			if (4 * ((size_t)nseg + 1) > rel_cap) {
+				mem.give(rel, rel_cap);
 				rel = nullptr;
-				rel_cap = nseg + 1;
-				SORTCHECK(hipMalloc(&rel, 4 * (size_t)rel_cap));
+				rel = (uint32_t*)mem.take(4 * ((size_t)nseg + 1), &rel_cap);
 			}
 			k_rel_offsets<<<(nseg + 256) / 256, 256, 0, s>>>(rowptr, r0, nseg, base, rel);
 			SORTCHECK(hipGetLastError());
 			size_t bytes = 0;
 			SORTCHECK(rocprim::segmented_radix_sort_keys(nullptr, bytes, in + base, out + base, size, nseg, rel,
 			                                             rel + 1, 0, (unsigned)bits, s));
-			if (bytes > tmp_bytes) {
-				if (tmp)
-					SORTCHECK(hipFree(tmp));
+			if (!tmp || bytes > tmp_cap) {
+				mem.give(tmp, tmp_cap);
 				tmp = nullptr;
-				tmp_bytes = bytes;
-				SORTCHECK(hipMalloc(&tmp, tmp_bytes));
+				tmp = mem.take(bytes, &tmp_cap);
 			}
 			SORTCHECK(rocprim::segmented_radix_sort_keys(tmp, bytes, in + base, out + base, size, nseg, rel, rel + 1,
 			                                             0, (unsigned)bits, s));
@@ -79,16 +74,12 @@ void sort_row_columns(const uint32_t* in, uint32_t* out, uint64_t nnz, uint32_t 
 		}
 	} catch (...) {
 		(void)hipStreamSynchronize(s);
-		if (rel)
-			(void)hipFree(rel);
-		if (tmp)
-			(void)hipFree(tmp);
+		mem.give(rel, rel_cap);
+		mem.give(tmp, tmp_cap);
 		throw;
 	}
-	if (rel)
-		SORTCHECK(hipFree(rel));
-	if (tmp)
-		SORTCHECK(hipFree(tmp));
+	mem.give(rel, rel_cap);
+	mem.give(tmp, tmp_cap);
 }
 
 } // namespace lgx
