@@ -964,7 +964,7 @@ def c4_extras(lib, leg, nth, cpu_seconds, with_cpu, n_patches=65536, bounces=4):
 
 def whole_scene_radiosity(lib, leg, tris, rng):
     """The bake's radiosity stage at C4's full size: links among all
-    11,917,038 texels (Int_RDGenLinks' pairs, found on the uniform grid, the
+    11,917,038 texels (Int_RDGenLinks' pairs, found over clusters, the
     CSR with 64-bit row offsets) and one bounce over them for one RGB setup
     (diffuse 0.6, world area per texel, seeded emission)."""
     S = len(leg.pos)
