@@ -3,6 +3,7 @@
 // pipeline and by the lgx_* entry points.
 #pragma once
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <stddef.h>
@@ -37,7 +38,8 @@ struct DevLight {
 };
 
 // Work items the allocation-free direct-light pass takes at most: its
-// scratch array holds 8 bytes per item (32 MiB) plus a few KiB.
+// scratch array holds 8 bytes per item (32 MiB), the list of long marches and
+// a few KiB.
 constexpr size_t kNoAllocMaxItems = (size_t)1 << 22;
 // GPUs per process whose scratch address is kept.
 constexpr int kMaxDevices = 64;
@@ -290,10 +292,9 @@ private:
 	float* d_gate_ = nullptr;     // shading factor per item (marched items)
 	uint32_t* d_mlist_ = nullptr; // compacted march list
 	uint32_t* d_mcount_ = nullptr; // [0] march count, then the march kernels' control words
-	void* d_long_ = nullptr;       // marches handed from a lane to a wave
 	uint32_t nmarch_ = 0;
 	unsigned persistent_blocks();
-	unsigned persist_blocks_ = 0;
+	std::atomic<unsigned> persist_blocks_{0};
 	std::vector<DevLight> h_lights_;
 	std::vector<uint32_t> h_light_off_;
 	size_t nitems_ = 0;

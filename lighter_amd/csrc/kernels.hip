@@ -2634,18 +2634,19 @@ template <class T> struct Scratch {
 // ---------------------------------------------------------------------------
 // Scratch of the allocation-free direct-light pass (run_direct_noalloc): the
 // buffers run_direct allocates (per-item shading factor, the march list, the
-// march count and list cursor, the traversal counters, the lights and their
-// item ranges) carved out of one file-scope device array.  Each GPU holds
-// its own copy for the life of the process; every call on a GPU uses that
-// copy, so calls that overlap on one GPU race.
+// march count and control words, the traversal counters, the lights and their
+// item ranges, the list of long marches) carved out of one file-scope device
+// array.  Each GPU holds its own copy for the life of the process; every call
+// on a GPU uses that copy, so calls that overlap on one GPU race.
 // ---------------------------------------------------------------------------
 constexpr size_t kNoAllocGateOff = 0;                                          // float per item
 constexpr size_t kNoAllocListOff = kNoAllocGateOff + 4 * kNoAllocMaxItems;      // uint32 per item
-constexpr size_t kNoAllocHeadOff = kNoAllocListOff + 4 * kNoAllocMaxItems;      // count, cursor, bad-item flag
+constexpr size_t kNoAllocHeadOff = kNoAllocListOff + 4 * kNoAllocMaxItems;      // march count, control words, bad-item flag
 constexpr size_t kNoAllocCntOff = kNoAllocHeadOff + 256;                        // traversal counters
 constexpr size_t kNoAllocLightOff = kNoAllocCntOff + 256;                       // 64 lights
 constexpr size_t kNoAllocOffOff = kNoAllocLightOff + 64 * sizeof(DevLight);     // 65 item offsets
-constexpr size_t kNoAllocBytes = kNoAllocOffOff + 512;
+constexpr size_t kNoAllocLongOff = kNoAllocOffOff + 512;                        // long marches
+constexpr size_t kNoAllocBytes = kNoAllocLongOff + kLongCap * sizeof(LongMarch);
 static_assert(kNumCounters * 8 <= 256, "counters fit their slot");
 static_assert(kNoAllocLightOff % 256 == 0 && kNoAllocOffOff % 256 == 0, "aligned slots");
 
@@ -2700,7 +2701,6 @@ DeviceScene::DeviceScene()
 	stream_ = s;
 	d_counters_ = dalloc<unsigned long long>(kNumCounters);
 	d_mcount_ = dalloc<uint32_t>(1 + kMarchWords + 6); // + the samples' bounds
-	d_long_ = dalloc<LongMarch>(kLongCap);
 	d_scratch_ = noalloc_scratch();
 	// the march's abort flag and progress word: pinned, coherent host memory
 	// the kernel reads and writes while it runs
@@ -2719,7 +2719,7 @@ size_t DeviceScene::march_lds_bytes() const { return (size_t)kBlock * march_stac
 
 unsigned DeviceScene::persistent_blocks()
 {
-	if (!persist_blocks_) {
+	if (!persist_blocks_) { // calls that overlap may both find it so: they store the same value
 		int dev = 0, per_cu = 0;
 		hipDeviceProp_t p;
 		HIPCHECK(hipGetDevice(&dev));
@@ -2732,7 +2732,9 @@ unsigned DeviceScene::persistent_blocks()
 }
 
 // Launches the marches of src (nmarch of them) on the stream; next: the
-// control words, zeroed on the stream but for an abort flag.  Up to
+// control words, zeroed on the stream but for an abort flag, and lng: the
+// list of long marches, both the launch's own while it runs (neither is
+// touched at up to Src::kWaveMax marches that cannot be stopped).  Up to
 // Src::kWaveMax marches take a wave each from the start: that few leave a
 // lane's marches waiting on the slowest walk of its wave, about 16 us a step
 // (128,001 items of a room, 87,091 marches: 1,156 us with waves, 1,198 us on
@@ -2745,7 +2747,7 @@ unsigned DeviceScene::persistent_blocks()
 // stated on.
 constexpr uint32_t kLongSteps = 64, kTailSteps = 64;
 template <class Src>
-static void launch_marches(const View& V, const Src& src, uint32_t nmarch, uint32_t* next, void* lng,
+static void launch_marches(const View& V, const Src& src, uint32_t nmarch, uint32_t* next, LongMarch* lng,
                            unsigned long long* cnt, bool counting, int depth, size_t lds, unsigned blocks, uint32_t* ctl,
                            hipStream_t s)
 {
@@ -2757,10 +2759,9 @@ static void launch_marches(const View& V, const Src& src, uint32_t nmarch, uint3
 		k_march_wave<<<std::min((nmarch + per - 1) / per, blocks), kBlock, lds, s>>>(V, src, nmarch, nullptr, nullptr,
 		                                                                              stop, depth);
 	} else {
-		k_march<false><<<blocks, kBlock, lds, s>>>(V, src, nmarch, next, cnt, depth, ctl, kLongSteps, kTailSteps,
-		                                           (LongMarch*)lng);
+		k_march<false><<<blocks, kBlock, lds, s>>>(V, src, nmarch, next, cnt, depth, ctl, kLongSteps, kTailSteps, lng);
 		HIPCHECK(hipGetLastError());
-		k_march_wave<<<blocks, kBlock, lds, s>>>(V, src, 0, (const LongMarch*)lng, next + kMarchLong, stop, depth);
+		k_march_wave<<<blocks, kBlock, lds, s>>>(V, src, 0, lng, next + kMarchLong, stop, depth);
 	}
 	HIPCHECK(hipGetLastError());
 }
@@ -2770,7 +2771,6 @@ DeviceScene::~DeviceScene()
 	free_all();
 	dfree(d_counters_);
 	dfree(d_mcount_);
-	dfree(d_long_);
 	if (stream_)
 		(void)hipStreamDestroy((hipStream_t)stream_);
 	if (ctl_host_)
@@ -3273,13 +3273,14 @@ bool DeviceScene::run_direct(const std::function<bool(float)>& keep_going)
 		HIPCHECK(hipMemcpyAsync(&nmarch, d_mcount_, 4, hipMemcpyDeviceToHost, s));
 		HIPCHECK(hipStreamSynchronize(s));
 		nmarch_ = nmarch;
+		Scratch<LongMarch> lng(spare_, nmarch > DirectSrc::kWaveMax ? kLongCap : 0);
 		EventTimer tm(s);
 		if (nmarch) {
 			// the abort and progress path only for runs that can be stopped
 			// (it costs up to 2 % of the march on the city block)
 			uint32_t* ctl = (keep_going || abort_requested_) ? ctl_dev_ : nullptr;
 			const DirectSrc src{d_pos_, d_nrm_, d_lights_, d_items_, d_mlist_, d_gate_, d_w_, d_vis_};
-			launch_marches(V, src, nmarch, d_mcount_ + 1, d_long_, d_counters_, count_queries, march_stack_depth(),
+			launch_marches(V, src, nmarch, d_mcount_ + 1, lng.p, d_counters_, count_queries, march_stack_depth(),
 			               march_lds_bytes(), persistent_blocks(), ctl, s);
 			aborted = wait_march(nmarch, keep_going);
 		}
@@ -3370,7 +3371,7 @@ void DeviceScene::run_direct_noalloc(const DevLight* lights, int nlights, const 
 	const uint32_t nmarch = h[0];
 	if (nmarch) {
 		const DirectSrc src{d_pos_, d_nrm_, dl, d_items, mlist, gate, d_w, d_vis};
-		launch_marches(V, src, nmarch, head + 1, d_long_, cnt, false, march_stack_depth(), march_lds_bytes(),
+		launch_marches(V, src, nmarch, head + 1, (LongMarch*)(sc + kNoAllocLongOff), cnt, false, march_stack_depth(), march_lds_bytes(),
 		               persistent_blocks(), nullptr, s);
 	}
 	for (int l = 0; l < nlights; ++l) {
@@ -3868,12 +3869,18 @@ void DeviceScene::query_shadow(const float* from, const float* to, const float* 
 	HIPCHECK(hipMemcpy(dk, k, 4 * n, hipMemcpyHostToDevice));
 	hipStream_t s = (hipStream_t)stream_;
 	const size_t chunk = size_t(1) << 30; // the list cursor is 32-bit
+	// control words and list of this call's own: other calls on this device
+	// scene may overlap it, and k_march's claims and hand-overs are theirs
+	const bool lanes = n > QuerySrc::kWaveMax;
+	Scratch<uint32_t> words(spare_, lanes ? kMarchWords : 0);
+	Scratch<LongMarch> lng(spare_, lanes ? kLongCap : 0);
 	size_t b = 0;
 	do {
 		const uint32_t m = (uint32_t)std::min(n - b, chunk);
-		k_fill_u32<<<1, 64, 0, s>>>(d_mcount_, 1 + kMarchWords, 0u);
+		if (lanes)
+			k_fill_u32<<<1, 64, 0, s>>>(words.p, kMarchWords, 0u);
 		const QuerySrc src{da + 3 * b, db + 3 * b, dk + b, dout + b, dst + b};
-		launch_marches(V, src, m, d_mcount_ + 1, d_long_, nullptr, false, march_stack_depth(), march_lds_bytes(),
+		launch_marches(V, src, m, words.p, lng.p, nullptr, false, march_stack_depth(), march_lds_bytes(),
 		               persistent_blocks(), nullptr, s);
 		b += m;
 	} while (b < n);
