@@ -191,7 +191,7 @@ LTRAPI int lgx_DeviceAbort(lgx_Device* dev, int on);
  * and the weights and factors are those lgx_ReadWeights would return.  The
  * kernels' scratch (per-item shading factors, the march list, counters, the
  * long marches) is a file-scope device array for 4,194,304 work items
- * (33.3 MiB), one per GPU for the life of the process: more items are refused, and calls
+ * (42 MiB), one per GPU for the life of the process: more items are refused, and calls
  * that overlap on one GPU race on it.  Synchronous. */
 LTRAPI int lgx_DirectLightNoAlloc(lgx_Device* dev, const lgx_Light* lights, int nlights, const uint32_t* d_items,
                                   size_t nitems, const uint32_t* light_off, float* d_weights, float* d_vis);

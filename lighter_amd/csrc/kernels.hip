@@ -917,7 +917,12 @@ struct LongMarch {
 };
 // Words of a march's control block (zeroed before the launches).
 constexpr int kMarchCursor = 0, kMarchAbort = 1, kMarchLong = 2, kMarchWords = 3;
-constexpr uint32_t kLongCap = 1u << 16; // marches that can be handed over (20 bytes each); a lane keeps the rest
+// Marches that can be handed over (20 bytes each, 10 MiB); a lane keeps the
+// rest and asks no more.  As many as the lanes of a launch, and more than any
+// measured one hands over (107,000 of a city's 1.6 M): with a full list it is
+// the first to get there, not the longest, that went to waves (156,588 over
+// a list of 131,072: 18.2 ms instead of 12.0).
+constexpr uint32_t kLongCap = 1u << 19;
 
 // Persistent shadow-march kernel: every lane pulls a new march from the list
 // as soon as its current one ends (one atomic per wave per refill), so the
@@ -929,11 +934,11 @@ constexpr uint32_t kLongCap = 1u << 16; // marches that can be handed over (20 b
 // (abort), so every wave stops within one claim of the first such post.  (A variant that
 // interleaves single traversal actions of all lanes in one loop measured
 // 37% slower on the terrain workload.)
-// A march of more than limit steps, or of more than tail steps once the
-// list is empty, goes to the list of long marches (lng, kLongCap entries at
-// most), which k_march_wave finishes with a wave for each: a lane takes
-// about 4.5 us for a step, so one march of 1,791 steps along a wall kept a
-// launch of 161,236 marches (mean 28 steps) running for 8.1 ms.
+// A march of limit steps or more, or of tail steps once the list is empty
+// (looked at every 16 steps), goes to the list of long marches (lng), which
+// k_march_wave finishes with a wave for each: a lane takes about 4.5 us for a
+// step, so one march of 1,791 steps along a wall kept a launch of 161,236
+// marches (mean 28 steps) running for 8.1 ms.
 // The traversal stack's first levels live in LDS (dynamic, kBlock * depth * 6
 // bytes: an int32 reference and an FP16 key per level and lane), depth =
 // min(kLdsLevels, levels of the BVH plus margin).
@@ -1015,6 +1020,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 				if (at < kLongCap) {
 					lng[at] = LongMarch{k, M.t, M.res, M.radius, M.steps};
 					active = false;
+				} else {
+					limit = tail = UINT32_MAX;
 				}
 			}
 		}
@@ -2739,13 +2746,22 @@ unsigned DeviceScene::persistent_blocks()
 // lane's marches waiting on the slowest walk of its wave, about 16 us a step
 // (128,001 items of a room, 87,091 marches: 1,156 us with waves, 1,198 us on
 // lanes; 8,001 items: 250 us and 1,100 us).  More keep the lanes busy, and
-// only the long ones go to waves: from 64 steps on, of which the last step
-// of a launch's last lanes is one (direct light on a city, 161,236 marches:
-// 2.06 ms with 64, 2.1 ms with 32, where the terrain's 917,990 marches
-// overflow the list of long ones: 6.4 and 8.2 ms; 8.4 and 7.8 ms without).
+// only marches that would hold the launch up go to waves: while the list
+// lasts, those longer than what a lane marches in all (kShareSteps steps for
+// each march that falls to it), as beside shorter ones it has other work; at
+// the end, those of kTailSteps steps.  A pass in ms, by the first limit (the
+// rule's choice in brackets, "-" for none) and without hand-over:
+//   marches                  64    96    128   192   -     none
+//   terrain 1.29 M  [79]    7.36  7.41  7.65  7.49  7.75
+//   city    1.60 M  [98]    8.43  8.09  8.16  8.11  8.08
+//   city    2.07 M [126]   12.0  11.2  11.2  11.1  11.2   19.3
+//   terrain 3.80 M [232]   18.4  17.1  16.7  16.4  16.5   19.9
+// kTailSteps, with no first limit: city of 2.07 M 16 steps 15.0, 32 12.1, 64
+// 11.3, 128 11.0; a room of 161,931 items 0.83 (32), 1.12 (64), 1.48 (128),
+// 1.77 (none); 500,001 grazing queries in a terrain 7.2, 5.3, 5.5, 6.0.
 // With counters every march stays on its lane, whose walk the counters are
 // stated on.
-constexpr uint32_t kLongSteps = 64, kTailSteps = 64;
+constexpr uint32_t kShareSteps = 24, kTailSteps = 64;
 template <class Src>
 static void launch_marches(const View& V, const Src& src, uint32_t nmarch, uint32_t* next, LongMarch* lng,
                            unsigned long long* cnt, bool counting, int depth, size_t lds, unsigned blocks, uint32_t* ctl,
@@ -2759,7 +2775,9 @@ static void launch_marches(const View& V, const Src& src, uint32_t nmarch, uint3
 		k_march_wave<<<std::min((nmarch + per - 1) / per, blocks), kBlock, lds, s>>>(V, src, nmarch, nullptr, nullptr,
 		                                                                              stop, depth);
 	} else {
-		k_march<false><<<blocks, kBlock, lds, s>>>(V, src, nmarch, next, cnt, depth, ctl, kLongSteps, kTailSteps, lng);
+		const uint64_t share = (uint64_t)kShareSteps * nmarch / (blocks * kBlock);
+		k_march<false><<<blocks, kBlock, lds, s>>>(V, src, nmarch, next, cnt, depth, ctl,
+		                                           (uint32_t)std::max<uint64_t>(kTailSteps, share), kTailSteps, lng);
 		HIPCHECK(hipGetLastError());
 		k_march_wave<<<blocks, kBlock, lds, s>>>(V, src, 0, lng, next + kMarchLong, stop, depth);
 	}

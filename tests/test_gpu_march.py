@@ -34,6 +34,33 @@ def soup(kind, rng):
 
 @pytest.mark.parametrize("kind", ["crowd", "walls", "far", "empty"])
 def test_wave_and_lane_marches_agree(lib, kind):
+    dev, a, b, k = workload(lib, kind)
+    one, steps = dev.shadow(a, b, k)
+    many, steps2 = dev.shadow(np.tile(a, (COPIES, 1)), np.tile(b, (COPIES, 1)), np.tile(k, COPIES))
+    dev.close()
+    many, steps2 = many.reshape(COPIES, N), steps2.reshape(COPIES, N)
+    same = (many.view(np.uint32) == one.view(np.uint32)).all(0) & (steps2 == steps).all(0)
+    assert same.all(), (kind, np.flatnonzero(~same)[:5], one[~same][:5], many[0][~same][:5])
+    if kind == "walls":
+        assert steps.max() > 128  # some were handed over
+
+
+def test_more_long_marches_than_the_list_holds(lib):
+    """A launch whose every march is long: more of them reach the limit than
+    the list of long marches takes (524,288)."""
+    dev, a, b, k = workload(lib, "walls")
+    one, steps = dev.shadow(a, b, k)
+    at = np.flatnonzero(steps >= 96)
+    assert len(at) >= 8
+    at = np.resize(at, 700_000)
+    many, steps2 = dev.shadow(a[at], b[at], k[at])
+    dev.close()
+    assert np.array_equal(many.view(np.uint32), one[at].view(np.uint32))
+    assert np.array_equal(steps2, steps[at])
+
+
+def workload(lib, kind):
+    """The device and N marches on it: from, to, k."""
     rng = np.random.default_rng(len(kind))
     tris, ext = soup(kind, rng)
     tris = tris.astype(np.float32).reshape(-1, 9)
@@ -51,12 +78,4 @@ def test_wave_and_lane_marches_agree(lib, kind):
         b[:n] = p + (t[:, 1] - t[:, 0]) * rng.uniform(1, 4, (n, 1)) + 0.02 * nrm
     b[-1] = a[-1]
     k = rng.choice([0.0, -0.1, 1e-3, 0.05, 0.5, 3.0], N).astype(np.float32)
-    dev = Device(lib, tris)
-    one, steps = dev.shadow(a, b, k)
-    many, steps2 = dev.shadow(np.tile(a, (COPIES, 1)), np.tile(b, (COPIES, 1)), np.tile(k, COPIES))
-    dev.close()
-    many, steps2 = many.reshape(COPIES, N), steps2.reshape(COPIES, N)
-    same = (many.view(np.uint32) == one.view(np.uint32)).all(0) & (steps2 == steps).all(0)
-    assert same.all(), (kind, np.flatnonzero(~same)[:5], one[~same][:5], many[0][~same][:5])
-    if kind == "walls":
-        assert steps.max() > 128  # some were handed over
+    return Device(lib, tris), a, b, k
