@@ -923,6 +923,7 @@ constexpr int kMarchCursor = 0, kMarchAbort = 1, kMarchLong = 2, kMarchWords = 3
 // the first to get there, not the longest, that went to waves (156,588 over
 // a list of 131,072: 18.2 ms instead of 12.0).
 constexpr uint32_t kLongCap = 1u << 19;
+constexpr int kFewLong = 48;
 
 // Persistent shadow-march kernel: every lane pulls a new march from the list
 // as soon as its current one ends (one atomic per wave per refill), so the
@@ -938,7 +939,14 @@ constexpr uint32_t kLongCap = 1u << 19;
 // (looked at every 16 steps), goes to the list of long marches (lng), which
 // k_march_wave finishes with a wave for each: a lane takes about 4.5 us for a
 // step, so one march of 1,791 steps along a wall kept a launch of 161,236
-// marches (mean 28 steps) running for 8.1 ms.
+// marches (mean 28 steps) running for 8.1 ms.  A wave of which more than
+// kFewLong lanes march long keeps them: its lanes are all at work and mostly
+// on the same nodes (a plane under a grazing sun, 260,100 marches of
+// thousands of steps each: 285 ms handed over, 102 kept; 500,001 grazing
+// queries in a room 2.78 and 2.46 ms).  With 16 in place of 48 the waves that
+// hold several of a city's long marches keep them too long (2.07 M marches
+// 13.5 ms instead of 11.1; 32: 11.1, and a terrain of 1.29 M 7.9 instead of
+// 7.5).
 // The traversal stack's first levels live in LDS (dynamic, kBlock * depth * 6
 // bytes: an int32 reference and an FP16 key per level and lane), depth =
 // min(kLdsLevels, levels of the BVH plus margin).
@@ -1007,6 +1015,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 		}
 		if (__all(done))
 			break;
+		// as it will be after the step
+		const bool few = !COUNT && __popcll(__ballot(active && M.steps + 1 >= limit)) <= kFewLong;
 		if (active) {
 			if (march_step(M, [&](f3 p, float R) { return q_distance<COUNT>(V, p, R, cnt, st); })) {
 				src.finish(M, k);
@@ -1015,7 +1025,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 					atomicAdd(cnt + 4, 1ull);
 				}
 				active = false;
-			} else if (!COUNT && M.steps >= limit && (M.steps & 15u) == 0) {
+			} else if (few && M.steps >= limit && (M.steps & 15u) == 0) {
 				const uint32_t at = atomicAdd(next + kMarchLong, 1u);
 				if (at < kLongCap) {
 					lng[at] = LongMarch{k, M.t, M.res, M.radius, M.steps};
