@@ -1211,9 +1211,8 @@ __device__ __forceinline__ void face_steps(March& M, f3 n, float d, float face)
 
 template <class Src>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_march_wave(View V, Src src, uint32_t nfresh,
-                                                       const LongMarch* __restrict__ lng,
-                                                       const uint32_t* __restrict__ nlng, const uint32_t* stop,
-                                                       int depth)
+                                                       const LongMarch* __restrict__ lng, uint32_t* next,
+                                                       uint32_t* ctl, int depth)
 {
 	extern __shared__ __align__(16) unsigned char lds_stack[];
 	__shared__ uint32_t queues[kBlock / 64][kGatherQueue], tris[kBlock / 64][64];
@@ -1221,13 +1220,28 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	uint32_t* queue = queues[wave];
 	uint32_t* tri = tris[wave];
-	const uint32_t n = lng ? min(*nlng, kLongCap) : nfresh;
+	const uint32_t n = lng ? (uint32_t)__builtin_amdgcn_readfirstlane((int)min(next[kMarchLong], kLongCap)) : nfresh;
 	// a fixed stride over the list: a claim per march on one counter would
 	// take longer than most marches here
 	const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + wave));
 	for (uint32_t idx = w0; idx < n; idx += gridDim.x * (kBlock / 64)) {
-		if (stop && __hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-			break;
+		// as k_march's claims: every march first reads the device's abort flag,
+		// one wave in 64 also the host's and posts the marches begun (64 for
+		// each of its own, a lane one; when they come from lng, all of them
+		// are).  The decision is the wave's: its lanes march together.
+		if (ctl) {
+			if ((w0 & 63u) == 0) {
+				if (!lng) {
+					const uint32_t begun = (uint32_t)__builtin_amdgcn_readfirstlane((int)atomicAdd(next + kMarchCursor, 1u));
+					__hip_atomic_store(ctl + 1, begun, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+				}
+				if (__hip_atomic_load(ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))
+					__hip_atomic_store(next + kMarchAbort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			}
+			if (__builtin_amdgcn_readfirstlane(
+			        (int)__hip_atomic_load(next + kMarchAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+				break;
+		}
 		March M;
 		const uint32_t k = lng ? lng[idx].key : src.key(idx);
 		src.init(M, V, k);
@@ -2778,18 +2792,17 @@ static void launch_marches(const View& V, const Src& src, uint32_t nmarch, uint3
                            hipStream_t s)
 {
 	constexpr unsigned per = kBlock / 64;
-	const uint32_t* stop = ctl ? next + kMarchAbort : nullptr;
 	if (counting) {
 		k_march<true><<<blocks, kBlock, lds, s>>>(V, src, nmarch, next, cnt, depth, ctl, UINT32_MAX, UINT32_MAX, nullptr);
 	} else if (nmarch <= Src::kWaveMax) {
-		k_march_wave<<<std::min((nmarch + per - 1) / per, blocks), kBlock, lds, s>>>(V, src, nmarch, nullptr, nullptr,
-		                                                                              stop, depth);
+		k_march_wave<<<std::min((nmarch + per - 1) / per, blocks), kBlock, lds, s>>>(V, src, nmarch, nullptr, next, ctl,
+		                                                                              depth);
 	} else {
 		const uint64_t share = (uint64_t)kShareSteps * nmarch / (blocks * kBlock);
 		k_march<false><<<blocks, kBlock, lds, s>>>(V, src, nmarch, next, cnt, depth, ctl,
 		                                           (uint32_t)std::max<uint64_t>(kTailSteps, share), kTailSteps, lng);
 		HIPCHECK(hipGetLastError());
-		k_march_wave<<<blocks, kBlock, lds, s>>>(V, src, 0, lng, next + kMarchLong, stop, depth);
+		k_march_wave<<<blocks, kBlock, lds, s>>>(V, src, 0, lng, next, ctl, depth);
 	}
 	HIPCHECK(hipGetLastError());
 }
@@ -3261,6 +3274,7 @@ bool DeviceScene::wait_march(uint32_t nmarch, const std::function<bool(float)>& 
 	hipStream_t s = (hipStream_t)stream_;
 	volatile uint32_t* ctl = ctl_host_;
 	bool stop = false;
+	float done = 0.0f; // posts of different waves may arrive in another order
 	for (;;) {
 		const hipError_t e = hipStreamQuery(s);
 		if (e == hipSuccess)
@@ -3268,8 +3282,8 @@ bool DeviceScene::wait_march(uint32_t nmarch, const std::function<bool(float)>& 
 		if (e != hipErrorNotReady)
 			HIPCHECK(e);
 		if (!stop) {
-			const float f = std::min(1.0f, (float)ctl[1] / (float)nmarch);
-			if (!keep_going(f)) {
+			done = std::max(done, std::min(1.0f, (float)ctl[1] / (float)nmarch));
+			if (!keep_going(done)) {
 				stop = true;
 				ctl[0] = 1u;
 			}

@@ -13,12 +13,13 @@ before.
 (The stage-boundary abort of a whole bake runs on the CPU in test_abi.py.)
 """
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
 
 from helpers import Device, P, all_samples_and_tris, bits, prepared
-from lighter_amd import _lib, scenes, workloads
+from lighter_amd import _lib, api, scenes, workloads
 
 pytestmark = pytest.mark.gpu
 u32p = C.POINTER(C.c_uint32)
@@ -71,3 +72,56 @@ def test_device_abort_stops_the_march_and_leaves_the_lightmap(lib):
     assert np.all(lm2 >= lm1) and np.any(lm2 > lm1)  # the second run added its light
     dev.close()
     b.destroy()
+
+
+def _grazing(extent, lm):
+    """A flat square of extent m under a sun 0.02 degrees above its plane: every
+    texel's march creeps thousands of steps along it, a wave's for
+    milliseconds."""
+    chart = scenes.Chart(np.zeros(3), np.array([extent, 0.0, 0.0]), np.array([0.0, extent, 0.0]), 1, 1, 0)
+    parts = scenes.charts_to_part_arrays([chart], lm, lm)
+    mesh = scenes.Mesh("ground", parts, [scenes.Instance(scenes.IDENTITY.copy(), 1.0, 1, "ground0")])
+    d = np.array([1.0, 0.3, 3e-4])
+    sun = scenes.dir_light(d / np.linalg.norm(d), np.ones(3), 2.0 * extent)
+    return scenes.SceneSpec("ground", [mesh], [sun], dict(bounce_count=0, blur_size=0.0, max_num_threads=4), lm_size=lm)
+
+
+def _bake(lib, spec, abort):
+    """Seconds from the first look at the running light stage (with abort:
+    from ltr_Abort then) to the bake's end, and the fractions seen between."""
+    b = scenes.BuiltScene(lib, spec)
+    st = api.WorkStatus()
+    seen, t0 = [], None
+    lib.ltr_Start(b.scene)
+    while lib.ltr_GetStatus(b.scene, C.byref(st)):
+        if st.stage == b"rendering lightmaps":
+            if t0 is None:
+                # a few looks: the march has begun
+                time.sleep(0.02)
+                t0 = time.perf_counter()
+                if abort:
+                    lib.ltr_Abort(b.scene)
+            seen.append(st.completion)
+        time.sleep(0.0005)
+    t = time.perf_counter() - t0
+    outputs = len(b.outputs())
+    b.destroy()
+    return t, seen, outputs
+
+
+@pytest.mark.parametrize("extent,lm", [(2000.0, 256), (700.0, 512)])
+def test_abort_and_progress_of_a_bake_inside_a_march(lib, extent, lm):
+    """At most 65,536 marches, a wave for each from the start, which takes its
+    next ones while the stage runs: the fraction rises and ltr_Abort ends the
+    stage long before its time.  262,144 marches, all begun by lanes at once:
+    an abort still leaves the bake without outputs."""
+    spec = _grazing(extent, lm)
+    _bake(lib, spec, False)
+    full, seen, outputs = _bake(lib, spec, False)
+    assert outputs == 1 and full > 0.05, (full, outputs)
+    assert all(0.0 <= f <= 1.0 for f in seen) and seen == sorted(seen)
+    part, _, outputs = _bake(lib, spec, True)
+    assert outputs == 0
+    if lm == 256:
+        assert any(0.1 < f < 0.9 for f in seen), seen
+        assert part < 0.5 * full, (part, full)
