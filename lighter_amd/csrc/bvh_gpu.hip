@@ -29,6 +29,7 @@
 #include <string>
 #include <vector>
 
+#include "alloc.h"
 #include "bvh.h"
 
 namespace lgx {
@@ -74,7 +75,7 @@ template <class T> struct DArr {
 			(void)hipFree(p);
 		p = nullptr;
 		n = cnt;
-		BV_CHECK(hipMalloc((void**)&p, sizeof(T) * (cnt ? cnt : 1)));
+		p = (T*)device_alloc(sizeof(T) * cnt);
 	}
 	DArr(const DArr&) = delete;
 	DArr& operator=(const DArr&) = delete;

@@ -13,6 +13,8 @@
 #include <string>
 #include <vector>
 
+#include "alloc.h"
+
 namespace lgx {
 
 class SpareBlocks;
@@ -68,16 +70,17 @@ struct QueryCounters {
 };
 
 // Scratch blocks of one device scene, kept between its calls for the next
-// that asks for much the same size; at most 8 GiB of them, given back when an
-// allocation fails and with the scene.  All work on them is on the scene's
-// one stream (copies on the null stream wait for it), which orders a block's
-// next use after its last.
+// that asks for much the same size; at most 8 GiB of them, given back with
+// the scene and when any device allocation of the process fails
+// (device_alloc).  All work on them is on the scene's one stream (copies on
+// the null stream wait for it), which orders a block's next use after its
+// last.
 class SpareBlocks {
 public:
-	SpareBlocks() = default;
+	SpareBlocks();
 	SpareBlocks(const SpareBlocks&) = delete;
 	SpareBlocks& operator=(const SpareBlocks&) = delete;
-	~SpareBlocks() { release(); }
+	~SpareBlocks();
 	void* take(size_t bytes, size_t* cap);
 	void give(void* p, size_t cap);
 	void release();
@@ -86,6 +89,17 @@ private:
 	std::mutex mu_;
 	std::multimap<size_t, void*> spare_; // by size
 	size_t total_ = 0;
+};
+
+// an array from a scene's spare blocks, for one scope
+template <class T> struct Scratch {
+	SpareBlocks& from;
+	size_t cap = 0;
+	T* p;
+	Scratch(SpareBlocks& b, size_t n) : from(b), p((T*)b.take(n * sizeof(T), &cap)) {}
+	Scratch(const Scratch&) = delete;
+	Scratch& operator=(const Scratch&) = delete;
+	~Scratch() { from.give(p, cap); }
 };
 
 class DeviceScene {
@@ -245,6 +259,7 @@ public:
 	Rad rad;
 	size_t npatches = 0;
 	void* stream() const { return stream_; }
+	SpareBlocks& spare() { return spare_; } // for work on stream()
 
 private:
 	void free_all();

@@ -24,6 +24,7 @@
 #include <string>
 #include <thread>
 
+#include "alloc.h"
 #include "finalize.h"
 #include "texel.h"
 #include "vmath.h"
@@ -142,7 +143,7 @@ struct Pinned {
 
 struct Dev {
 	char* p = nullptr;
-	explicit Dev(size_t bytes) { FIN_CHECK(hipMalloc((void**)&p, bytes ? bytes : 1)); }
+	explicit Dev(size_t bytes) : p((char*)device_alloc(bytes)) {}
 	Dev(const Dev&) = delete;
 	Dev& operator=(const Dev&) = delete;
 	~Dev()

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <set>
 #include <stdexcept>
 #include <string>
 #include <thread>
@@ -2571,14 +2572,7 @@ std::string device_name()
 	return std::string(p.name) + " " + p.gcnArchName;
 }
 
-template <class T> static T* dalloc(size_t n)
-{
-	void* p = nullptr;
-	if (n == 0)
-		n = 1;
-	HIPCHECK(hipMalloc(&p, n * sizeof(T)));
-	return (T*)p;
-}
+template <class T> static T* dalloc(size_t n) { return (T*)device_alloc(n * sizeof(T)); }
 
 template <class T> static void dfree(T*& p)
 {
@@ -2603,6 +2597,52 @@ template <class T> struct DevArray {
 // 100,003 probe points: 2.44 -> 2.26 ms.
 constexpr size_t kSpareMax = size_t(8) << 30;
 
+// Every scene's spare blocks.  Blocks that a call holds are not among them,
+// and hipFree waits for the work on those it frees, so any thread may give
+// back another scene's.
+static std::mutex g_spares_mu;
+static std::set<SpareBlocks*>& spares()
+{
+	static std::set<SpareBlocks*>& all = *new std::set<SpareBlocks*>; // outlives any scene
+	return all;
+}
+
+SpareBlocks::SpareBlocks()
+{
+	std::lock_guard<std::mutex> g(g_spares_mu);
+	spares().insert(this);
+}
+
+SpareBlocks::~SpareBlocks()
+{
+	{
+		std::lock_guard<std::mutex> g(g_spares_mu);
+		spares().erase(this);
+	}
+	release();
+}
+
+void* device_alloc(size_t bytes)
+{
+	void* p = nullptr;
+	bytes = std::max<size_t>(bytes, 1);
+	if (hipMalloc(&p, bytes) == hipSuccess)
+		return p;
+	(void)hipGetLastError();
+	{
+		std::lock_guard<std::mutex> g(g_spares_mu);
+		for (SpareBlocks* s : spares())
+			s->release();
+	}
+	const hipError_t e = hipMalloc(&p, bytes);
+	if (e != hipSuccess) {
+		(void)hipGetLastError();
+		throw std::runtime_error(std::string("HIP error ") + hipGetErrorString(e) + ": allocating " +
+		                         std::to_string(bytes) + " bytes of device memory");
+	}
+	return p;
+}
+
 void* SpareBlocks::take(size_t bytes, size_t* cap)
 {
 	bytes = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
@@ -2617,12 +2657,7 @@ void* SpareBlocks::take(size_t bytes, size_t* cap)
 			return p;
 		}
 	}
-	void* p = nullptr;
-	if (hipMalloc(&p, bytes) != hipSuccess) {
-		(void)hipGetLastError();
-		release();
-		HIPCHECK(hipMalloc(&p, bytes));
-	}
+	void* p = device_alloc(bytes);
 	*cap = bytes;
 	return p;
 }
@@ -2650,17 +2685,6 @@ void SpareBlocks::release()
 	spare_.clear();
 	total_ = 0;
 }
-
-// an array from the scene's spare blocks, for one scope
-template <class T> struct Scratch {
-	SpareBlocks& from;
-	size_t cap = 0;
-	T* p;
-	Scratch(SpareBlocks& b, size_t n) : from(b), p((T*)b.take(n * sizeof(T), &cap)) {}
-	Scratch(const Scratch&) = delete;
-	Scratch& operator=(const Scratch&) = delete;
-	~Scratch() { from.give(p, cap); }
-};
 
 // ---------------------------------------------------------------------------
 // Scratch of the allocation-free direct-light pass (run_direct_noalloc): the

@@ -31,6 +31,7 @@
 #include <string>
 #include <thread>
 
+#include "alloc.h"
 #include "place.h"
 
 namespace lgx {
@@ -313,7 +314,7 @@ struct PinnedBlock {
 
 struct DevBlock {
 	char* p = nullptr;
-	explicit DevBlock(size_t bytes) { PLACE_CHECK(hipMalloc((void**)&p, bytes ? bytes : 1)); }
+	explicit DevBlock(size_t bytes) : p((char*)device_alloc(bytes)) {}
 	DevBlock(const DevBlock&) = delete;
 	DevBlock& operator=(const DevBlock&) = delete;
 	~DevBlock()

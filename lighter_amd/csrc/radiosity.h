@@ -65,8 +65,6 @@ private:
 	void apply_tiles_f32(const float* xT, float* yT, bool pre);
 	void apply_sparse(int form, const double* x, double* y, bool pre, double* tot = nullptr);
 	void grad_dense(int form, int B, const double* g, double* total, double* lam, double* dalb);
-	double* keep64(uint64_t n);
-	float* keep32(uint64_t n);
 	DeviceScene& dev;
 	void* s_ = nullptr;
 	float* g32_ = nullptr;
@@ -96,9 +94,6 @@ private:
 	float* part_ = nullptr;
 	float* xq_ = nullptr;
 	uint16_t* xqlo_ = nullptr;
-	float* keep32_ = nullptr; // iterates (column-major sets), the most a call needed
-	double* keep64_ = nullptr; // totals and the sweeps' vectors, the same
-	uint64_t keep32_n_ = 0, keep64_n_ = 0;
 	float* rmx_ = nullptr;  // sparse FP32 form: the operand (x diffuse) area prepared once per product
 	double* rmx64_ = nullptr; // the same for the FP64 form
 	unsigned* cmax_ = nullptr; // column maxima of the FP16 operand (its scales): two planes of kRPad

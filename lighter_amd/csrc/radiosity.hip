@@ -63,9 +63,7 @@ __device__ __forceinline__ int piece_swz(int row) { return ((row >> 1) ^ (row >>
 
 template <class T> static T* dalloc(size_t n)
 {
-	void* p = nullptr;
-	HIPCHECK(hipMalloc(&p, (n ? n : 1) * sizeof(T)));
-	return (T*)p;
+	return (T*)device_alloc(n * sizeof(T));
 }
 template <class T> static void dfree(T*& p)
 {
@@ -1347,8 +1345,6 @@ void RadSolver::release()
 	dfree(part_);
 	dfree(xq_);
 	dfree(xqlo_);
-	dfree(keep32_);
-	dfree(keep64_);
 	dfree(rmx_);
 	dfree(rmx64_);
 	dfree(cmax_);
@@ -1856,30 +1852,6 @@ void RadSolver::apply_sparse(int form, const double* x, double* y, bool pre, dou
 	HIPCHECK(hipGetLastError());
 }
 
-// n doubles (n floats of the iterates) kept across calls: allocating and
-// freeing them on every call cost more than a small problem's products.
-double* RadSolver::keep64(uint64_t n)
-{
-	if (n > keep64_n_) {
-		dfree(keep64_);
-		keep64_n_ = 0;
-		keep64_ = dalloc<double>(n);
-		keep64_n_ = n;
-	}
-	return keep64_;
-}
-
-float* RadSolver::keep32(uint64_t n)
-{
-	if (n > keep32_n_) {
-		dfree(keep32_);
-		keep32_n_ = 0;
-		keep32_ = dalloc<float>(n);
-		keep32_n_ = n;
-	}
-	return keep32_;
-}
-
 void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 {
 	chain_x_ = nullptr;
@@ -1891,7 +1863,11 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 	const uint64_t nR = (uint64_t)N * R, nRp = (uint64_t)R * Np;
 	times = RadTimes{};
 	ensure_work(form);
-	double* tot = keep64((form < kDenseF32 ? 3 : 1) * nR); // FP64 total
+	// the FP64 total (sparse forms: and two vectors) and the iterates are taken
+	// from the scene's spare blocks: allocating and freeing them on every call
+	// cost more than a small problem's products
+	Scratch<double> keep64(dev.spare(), (form < kDenseF32 ? 3 : 1) * nR);
+	double* tot = keep64.p;
 	if (form == kSparseF64 || form == kSparseF32) {
 		HIPCHECK(hipMemcpyAsync(tot, E_, 8 * nR, hipMemcpyDeviceToDevice, s));
 		const double* x = E_;
@@ -1909,7 +1885,8 @@ void RadSolver::solve(int form, int bounces, int refine, double* total_out)
 			build_dense(form);
 		times.build_ms = build_ms;
 		// z_k (column-major FP32), k = 0..b
-		float* z0 = keep32((uint64_t)(bounces + 1) * nRp);
+		Scratch<float> keep32(dev.spare(), (uint64_t)(bounces + 1) * nRp);
+		float* z0 = keep32.p;
 		std::vector<float*> z;
 		for (int b = 0; b <= bounces; ++b)
 			z.push_back(z0 + (uint64_t)b * nRp);
@@ -1984,7 +1961,8 @@ void RadSolver::solve_grad(int form, int bounces, const double* g, double* total
 	}
 	// row-major N x R sets: S_0 .. S_{B-1}, then the vectors of the sweeps
 	const uint64_t nS = std::max(1, B);
-	double* S = keep64((nS + 7) * nR);
+	Scratch<double> keep64(dev.spare(), (nS + 7) * nR);
+	double* S = keep64.p;
 	double *z = S + nS * nR, *zn = z + nR, *tot = zn + nR, *ybar = tot + nR, *u = ybar + nR, *lam = u + nR,
 	       *dalb = lam + nR;
 	Ev ev(s);
@@ -2034,9 +2012,11 @@ void RadSolver::grad_dense(int form, int B, const double* g, double* total_out, 
 	const float* diff = mo ? dperm_ : diff_;
 	const float* area = mo ? aperm_ : area_;
 	const uint32_t npos = mo ? Np : N;
-	double* S = keep64((uint64_t)(B + 3) * nRp + nR); // S_0 .. S_B, dalb, lam, then rows of the caller
+	Scratch<double> keep64(dev.spare(), (uint64_t)(B + 3) * nRp + nR); // S_0 .. S_B, dalb, lam, then rows of the caller
+	Scratch<float> keep32(dev.spare(), 2 * nRp);
+	double* S = keep64.p;
 	double *dalb = S + (uint64_t)(B + 1) * nRp, *lam = dalb + nRp, *rows = lam + nRp;
-	float *z = keep32(2 * nRp), *zn = z + nRp;
+	float *z = keep32.p, *zn = z + nRp;
 	Ev ev(s);
 	// forward: S_0 = E, z_k = K z_{k-1}, S_k = S_{k-1} + z_k
 	k_to_cols<double><<<tg, kB, 0, s>>>(E_, N, Np, R, po, S);

@@ -21,6 +21,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "alloc.h"
 #include "raster.h"
 #include "raster_gpu.h"
 
@@ -45,7 +46,7 @@ struct RasAtlas {
 
 template <class T> struct DevArr {
 	T* p = nullptr;
-	explicit DevArr(size_t n) { RAS_CHECK(hipMalloc((void**)&p, sizeof(T) * (n ? n : 1))); }
+	explicit DevArr(size_t n) : p((T*)device_alloc(sizeof(T) * n)) {}
 	DevArr(const DevArr&) = delete;
 	DevArr& operator=(const DevArr&) = delete;
 	~DevArr()

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from helpers import Device, P
+from hipmem import hip
 from lighter_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -39,4 +40,46 @@ def test_scratch_passes_between_calls(lib):
         one.close()
         for x, y in zip(*out):
             assert np.array_equal(x.view(np.uint32), y.view(np.uint32)), n
+    dev.close()
+
+
+def test_failed_allocation_gives_spare_blocks_back(lib):
+    """The scratch that one device keeps (1.6 GB after a query of 100 M
+    points) is there for a call of another that finds no memory: it is given
+    back before that call fails (a dense matrix of 360 GB here)."""
+    h = hip()
+    h.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+
+    def free_memory():
+        free, total = C.c_size_t(0), C.c_size_t(0)
+        assert h.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        assert total.value < 360e9
+        return free.value
+
+    rng = np.random.default_rng(12)
+    tris = rng.uniform(-3, 3, (20, 9)).astype(np.float32)
+
+    def dense_solve(n):
+        dev = Device(lib, tris)
+        pos = np.zeros((n, 3), np.float32)
+        pos[:, :2] = np.stack(np.divmod(np.arange(n), 1000), 1)
+        nrm = np.tile(np.array([0, 0, 1], np.float32), (n, 1))
+        nl = C.c_size_t(0)
+        _lib.check(lib.lgx_RadLinks(dev.h, P(pos), P(nrm), n, C.byref(nl)), lib)
+        E, diff, area = np.ones((n, 1)), np.ones((n, 3), np.float32), np.ones(n, np.float32)
+        dp = C.POINTER(C.c_double)
+        ok = lib.lgx_RadSolve(dev.h, E.ctypes.data_as(dp), 1, P(diff), P(area), 2, 1, 0,
+                              np.zeros_like(E).ctypes.data_as(dp), None)
+        dev.close()
+        return ok
+
+    assert dense_solve(1000) == 1
+    dev = Device(lib, tris)
+    dev.distance(np.zeros((1000, 3), np.float32))
+    before = free_memory()
+    dev.distance(np.zeros((100_000_000, 3), np.float32))
+    assert before - free_memory() > 1.5e9  # kept
+    assert dense_solve(300_000) == 0
+    assert "allocating" in _lib.last_error(lib)
+    assert before - free_memory() < 0.5e9
     dev.close()
