@@ -210,9 +210,10 @@ LTRAPI int lgx_AmbientOcclusion(lgx_Device* dev, const float* randoff, int num_s
  * the search falls back to all pairs. */
 LTRAPI int lgx_RadLinks(lgx_Device* dev, const float* pos3, const float* nrm3, size_t n, size_t* nlinks);
 /* No counterpart in the reference (tests). How the next lgx_RadLinks
- * finds its candidate pairs: modes 0 (default) and 2 among clusters of
- * patches, mode 1 all pairs, as the reference's loop does (at most 524,288
- * patches).  Every mode gives the same links. */
+ * finds its candidate pairs: mode 0 (default) all pairs of few patches (at
+ * most 6,144) and clusters of more, mode 1 all pairs, as the reference's
+ * loop does (at most 524,288 patches), mode 2 clusters.  Every mode gives the
+ * same links. */
 LTRAPI int lgx_SetLinkSearch(lgx_Device* dev, int mode);
 LTRAPI int lgx_RadReadLinks(lgx_Device* dev, uint32_t* rowmap, uint32_t* other, float* factor);
 /* bounce_count rounds of Int_RDBounce (lighter.cpp:767-797) from emitted

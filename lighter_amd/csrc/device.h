@@ -207,9 +207,10 @@ public:
 	// a shadow caster (the reference's VisibilityTest returns the hit).
 	// Candidates come from pairs of clusters of patches whose bounds allow a
 	// link, or from all pairs as the reference enumerates them (at most
-	// kMaxAllPairsPatches patches); both give the same links.  links_mode 0
-	// and 2: the clusters; 1: all pairs.  Patches with non-finite positions
-	// or normals always take all pairs.
+	// kMaxAllPairsPatches patches); both give the same links.  links_mode 0:
+	// all pairs of few patches, clusters of more; 1: all pairs; 2: the
+	// clusters.  Patches with non-finite positions or normals always take all
+	// pairs.
 	void rad_set_patches(const float* pos, const float* nrm, size_t n);
 	size_t rad_links();
 	int links_mode = 0;

@@ -2129,10 +2129,16 @@ __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, u
 // grid's candidate list (30.1 ms of pair tests, made twice; 12.6 ms of
 // occlusion tests on the list), 26 ms so (pair tests 2.4 ms); a room's 20 ->
 // 12 ms.
+// Where the patches are too few to fill the chip's waves, 2^split waves take a
+// patch, each a run of its cluster's partners, until there are kLinkWaves
+// (whole searches: a terrain of 3,001 patches 1.27 -> 0.70 ms, of 12,001 3.77
+// -> 2.60, a room of 6,001 1.43 -> 1.10; up to twice as many gained a terrain
+// of 32,768 6.24 -> 5.72 and lost a city of 32,768 2.05 -> 2.26).
 // mask: the candidates' bits in, the links' out.  cand, linked (optional): the
 // candidates and whether each linked, in any order from *ncand on.
 // The walk is one for the wave (wave_occluded).  Against a walk per lane: a room's
 // 12.7 -> 8.8 ms (25 G segments/s), a city's 16.4 -> 14.5 ms.
+constexpr uint32_t kLinkWaves = 32768, kLinkSplitMax = 4;
 struct LinkWave {
 	uint32_t stack[kStackSize];
 	uint32_t row[128]; // the candidates of 64 partners, from when they are queued on the links among them
@@ -2140,20 +2146,23 @@ struct LinkWave {
 };
 __global__ __launch_bounds__(kBlock) void k_cluster_links(
     View V, PairWork W, const uint64_t* __restrict__ first, const uint32_t* __restrict__ of,
-    uint64_t* __restrict__ mask, unsigned long long* ncand, uint2* __restrict__ cand, uint8_t* __restrict__ linked)
+    uint32_t split, uint64_t* __restrict__ mask, unsigned long long* ncand, uint2* __restrict__ cand,
+    uint8_t* __restrict__ linked)
 {
 	__shared__ LinkWave waves[kBlock / 64];
 	constexpr uint32_t per = kCl / (kBlock / 64); // blocks per cluster
 	const uint32_t lane = threadIdx.x & 63;
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-	const uint32_t a = blockIdx.x / per, i = blockIdx.x % per * (kBlock / 64) + wave;
+	const uint32_t a = (blockIdx.x / per) >> split, part = (blockIdx.x / per) & ((1u << split) - 1u);
+	const uint32_t i = blockIdx.x % per * (kBlock / 64) + wave;
 	const float4 A = W.sp[(size_t)a * kCl + i];
 	const uint32_t ia = __float_as_uint(A.w);
 	if (ia == kNoPatch)
 		return; // the whole wave; no block barrier below
 	LinkWave& L = waves[wave];
-	const uint64_t end = first[a + 1];
-	for (uint64_t p0 = first[a]; p0 < end; p0 += 64) {
+	const uint64_t begin = first[a], partners = first[a + 1] - begin;
+	const uint64_t end = begin + (partners * (part + 1) >> split);
+	for (uint64_t p0 = begin + (partners * part >> split); p0 < end; p0 += 64) {
 		uint64_t parts;
 		{
 			const uint64_t m = p0 + lane < end ? mask[(size_t)of[p0 + lane] * kCl + i] : 0;
@@ -4152,8 +4161,11 @@ uint64_t DeviceScene::links_by_clusters(uint32_t** colx, size_t* cap)
 		    npairs, at.p, nc, coff.p, pairs.p, pairs2.p, of.p, first2.p);
 		HIPCHECK(hipGetLastError());
 		if (nfull) {
-			k_cluster_links<<<nc * (kCl / (kBlock / 64)), kBlock, 0, s>>>(
-			    V, F, first2.p, of.p, mask.p, cursor.p, cand, linked);
+			uint32_t split = 0;
+			while (split < kLinkSplitMax && ((uint64_t)Npad << split) < kLinkWaves)
+				++split;
+			k_cluster_links<<<nc * (kCl / (kBlock / 64)) << split, kBlock, 0, s>>>(
+			    V, F, first2.p, of.p, split, mask.p, cursor.p, cand, linked);
 			HIPCHECK(hipGetLastError());
 			k_cluster_degrees<<<gridn_waves(nfull), kBlock, 0, s>>>(F, of.p, mask.p, deg.p);
 			HIPCHECK(hipGetLastError());
@@ -4215,6 +4227,13 @@ uint64_t DeviceScene::links_by_all_pairs(uint32_t** colx, size_t* cap)
 	return nnz;
 }
 
+// Up to so many patches the pairs are fewer than the clusters' launches and
+// waits are worth (ms, all pairs and clusters: 2 patches 0.18 and 0.28; 3,001
+// scattered in a city 0.49 and 0.85, in a row of a terrain 0.69 and 0.70, in
+// a room 0.76 and 0.73; 6,001 0.48 and 0.95, 1.10 and 1.15, 1.33 and 1.10;
+// 8,001 in a room 2.24 and 1.43).
+constexpr uint32_t kAllPairsBelow = 6144;
+
 size_t DeviceScene::rad_links()
 {
 	hipStream_t s = (hipStream_t)stream_;
@@ -4243,7 +4262,8 @@ size_t DeviceScene::rad_links()
 	// while they fit (the solver forms take those)
 	uint64_t nnz = 0;
 	if (N > 1) {
-		nnz = links_mode == 1 || !links_finite_ ? links_by_all_pairs(&colx, &colx_cap) : links_by_clusters(&colx, &colx_cap);
+		const bool all = links_mode == 1 || (links_mode == 0 && N <= kAllPairsBelow) || !links_finite_;
+		nnz = all ? links_by_all_pairs(&colx, &colx_cap) : links_by_clusters(&colx, &colx_cap);
 	} else {
 		HIPCHECK(hipMemsetAsync(rad.rowptr64, 0, 8 * ((size_t)N + 1), s));
 	}

@@ -51,10 +51,28 @@ def test_clusters_find_the_all_pairs_links(lib, kind, n):
     c = pos[rng.integers(0, n, 300)][:, None] + rng.uniform(-0.1, 0.1, (300, 1, 3)) * ext
     tris = (c + rng.uniform(-0.1, 0.1, (300, 3, 3)) * ext).astype(np.float32).reshape(-1, 9)
     dev = Device(lib, tris)
-    a, b = links(lib, dev, pos, nrm, 1), links(lib, dev, pos, nrm, 0)
+    a, b = links(lib, dev, pos, nrm, 1), links(lib, dev, pos, nrm, 2)
     dev.close()
     for x, y in zip(a, b):
         assert x.shape == y.shape
         assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
     if n >= 1000:  # only that there is something to compare (an unlinked set leaves one unused entry)
         assert len(a[1]) > 1
+
+
+@pytest.mark.parametrize("n", [2, 6144, 6145, 20_000])
+def test_automatic_choice_and_waves_per_patch(lib, n):
+    """Mode 0 on both sides of the count up to which it takes all pairs, and
+    the clusters with 16, 8 and 2 waves to a patch."""
+    rng = np.random.default_rng(n)
+    pos, nrm = patches("planes", n, rng)
+    pos[:, :2] += rng.uniform(0.0, 0.9, (n, 2)).astype(np.float32)
+    tris = rng.uniform(0.0, 24.0, (200, 9)).astype(np.float32)
+    tris[:, 2::3] *= 0.1
+    dev = Device(lib, tris)
+    a, b, c = (links(lib, dev, pos, nrm, m) for m in (1, 0, 2))
+    dev.close()
+    for x, y, z in zip(a, b, c):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+        assert np.array_equal(x.view(np.uint32), z.view(np.uint32))
+    assert n == 2 or len(a[1]) > 1000

@@ -1,16 +1,16 @@
-"""Radiosity link search: the uniform grid against the all-pairs enumeration.
+"""Radiosity link search: clusters of patches against the all-pairs
+enumeration.
 
-Int_RDGenLinks (lighter.cpp:728-759) tests every pair i < j.  A pair can
-only pass the factor threshold f = dA dB / (pi l^4) >= 0.001 when l^2 <=
-|nA| |nB| / (0.001 pi), so the product searches a uniform grid of cells that
-wide (every such pair lies in the same or a neighbouring cell) with the
-per-pair arithmetic of the all-pairs loop, and assembles the symmetric CSR
-by a per-row sort.  lgx_SetLinkSearch(dev, 1) switches to the all-pairs
-enumeration, mode 2 forces the grid, and the default takes all pairs where
-the grid would not prune.  Every mode must give the same links and factors
-bit for bit, also above 262,144 patches (where a pair bitmask would take
-N^2 / 8 = 8.6 GB); patches with non-finite positions or normals take the
-all-pairs path, whose links must then match the oracle's loop.
+Int_RDGenLinks (lighter.cpp:728-759) tests every pair i < j.  The product
+looks only at pairs of clusters of 64 patches whose boxes and normals allow
+a factor f = dA dB / (pi l^4) >= 0.001, with the per-pair arithmetic of the
+all-pairs loop, and assembles the symmetric CSR by a per-row sort.
+lgx_SetLinkSearch(dev, 1) switches to the all-pairs enumeration, mode 2 to
+the clusters, and the default takes all pairs of few patches.  Every mode
+must give the same links and factors bit for bit, also above 262,144 patches
+(where a pair bitmask would take N^2 / 8 = 8.6 GB); patches with non-finite
+positions or normals take the all-pairs path, whose links must then match the
+oracle's loop.
 """
 import ctypes as C
 
@@ -25,7 +25,7 @@ u32p = C.POINTER(C.c_uint32)
 
 
 def links(lib, dev, pos, nrm, mode):
-    """mode 0: automatic, 1: all pairs, 2: the grid"""
+    """mode 0: automatic, 1: all pairs, 2: clusters"""
     _lib.check(lib.lgx_SetLinkSearch(dev.h, mode), lib)
     nl = C.c_size_t(0)
     _lib.check(lib.lgx_RadLinks(dev.h, P(pos), P(nrm), len(pos), C.byref(nl)), lib)
@@ -47,7 +47,7 @@ SCENES = {
 
 
 @pytest.mark.parametrize("name", list(SCENES))
-def test_grid_search_finds_the_all_pairs_links(lib, name):
+def test_cluster_search_finds_the_all_pairs_links(lib, name):
     b = prepared(lib, SCENES[name]())
     pos, nrm, tris = all_samples_and_tris(lib, b)
     pn = scenes.normalize_rows_f32(nrm)
@@ -55,27 +55,27 @@ def test_grid_search_finds_the_all_pairs_links(lib, name):
         assert len(pos) > 262144
     dev = Device(lib, tris)
     try:
-        rm_g, ot_g, fa_g = links(lib, dev, pos, pn, 2)
+        rm_c, ot_c, fa_c = links(lib, dev, pos, pn, 2)
         rm_a, ot_a, fa_a = links(lib, dev, pos, pn, 1)
         rm_d, ot_d, fa_d = links(lib, dev, pos, pn, 0)
         assert np.array_equal(rm_d, rm_a) and np.array_equal(ot_d, ot_a)
-        print(f"{name}: {len(pos)} patches, {len(ot_g)} links")
-        assert len(ot_g) > 1000
-        assert np.array_equal(rm_g, rm_a)
-        assert np.array_equal(ot_g, ot_a)
-        assert np.array_equal(bits(fa_g), bits(fa_a))
+        print(f"{name}: {len(pos)} patches, {len(ot_c)} links")
+        assert len(ot_c) > 1000
+        assert np.array_equal(rm_c, rm_a)
+        assert np.array_equal(ot_c, ot_a)
+        assert np.array_equal(bits(fa_c), bits(fa_a))
         # rows list their links by ascending patch index, every factor passes
-        for i in np.flatnonzero(rm_g[1::2] > 1)[:2000]:
-            o, c = rm_g[2 * i], rm_g[2 * i + 1]
-            assert np.all(np.diff(ot_g[o:o + c].astype(np.int64)) > 0)
-        assert np.all(fa_g >= np.float32(0.001))
+        for i in np.flatnonzero(rm_c[1::2] > 1)[:2000]:
+            o, c = rm_c[2 * i], rm_c[2 * i + 1]
+            assert np.all(np.diff(ot_c[o:o + c].astype(np.int64)) > 0)
+        assert np.all(fa_c >= np.float32(0.001))
     finally:
         dev.close()
         b.destroy()
 
 
 def test_non_finite_normals_take_the_all_pairs_loop(lib, orc):
-    """A NaN normal and an infinite normal component: no cell width bounds
+    """A NaN normal and an infinite normal component: no box bounds
     such pairs, so the search enumerates all pairs, and their tests compare
     as the reference's do (NaN fails neither `<=` nor `<`, so the pair is
     tested for occlusion and links with a NaN factor; +inf links with an
