@@ -2135,7 +2135,7 @@ __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, u
 // -> 2.60, a room of 6,001 1.43 -> 1.10; up to twice as many gained a terrain
 // of 32,768 6.24 -> 5.72 and lost a city of 32,768 2.05 -> 2.26).
 // mask: the candidates' bits in, the links' out.  cand, linked (optional): the
-// candidates and whether each linked, in any order from *ncand on.
+// candidates and whether each linked, a wave's from its candoff on.
 // The walk is one for the wave (wave_occluded).  Against a walk per lane: a room's
 // 12.7 -> 8.8 ms (25 G segments/s), a city's 16.4 -> 14.5 ms.
 constexpr uint32_t kLinkWaves = 32768, kLinkSplitMax = 4;
@@ -2146,7 +2146,7 @@ struct LinkWave {
 };
 __global__ __launch_bounds__(kBlock) void k_cluster_links(
     View V, PairWork W, const uint64_t* __restrict__ first, const uint32_t* __restrict__ of,
-    uint32_t split, uint64_t* __restrict__ mask, unsigned long long* ncand, uint2* __restrict__ cand,
+    uint32_t split, uint64_t* __restrict__ mask, const uint64_t* __restrict__ candoff, uint2* __restrict__ cand,
     uint8_t* __restrict__ linked)
 {
 	__shared__ LinkWave waves[kBlock / 64];
@@ -2162,6 +2162,7 @@ __global__ __launch_bounds__(kBlock) void k_cluster_links(
 	LinkWave& L = waves[wave];
 	const uint64_t begin = first[a], partners = first[a + 1] - begin;
 	const uint64_t end = begin + (partners * (part + 1) >> split);
+	uint64_t at = cand ? candoff[blockIdx.x * (kBlock / 64) + wave] : 0;
 	for (uint64_t p0 = begin + (partners * part >> split); p0 < end; p0 += 64) {
 		uint64_t parts;
 		{
@@ -2201,14 +2202,13 @@ __global__ __launch_bounds__(kBlock) void k_cluster_links(
 				atomicOr(&L.row[e >> 5], 1u << (e & 31u));
 			}
 			if (cand) {
-				unsigned long long at = 0;
 				if (lane < n) {
-					at = atomicAdd(ncand, 1ull);
 					const uint32_t e = L.queue[lane];
 					const uint32_t ib = __float_as_uint(W.sp[(size_t)W.pairs[p0 + (e >> 6)].y * kCl + (e & 63u)].w);
-					cand[at] = make_uint2(min(ia, ib), max(ia, ib));
-					linked[at] = l ? 1 : 0;
+					cand[at + lane] = make_uint2(min(ia, ib), max(ia, ib));
+					linked[at + lane] = l ? 1 : 0;
 				}
+				at += n;
 			}
 			const uint16_t rest = L.queue[64 + lane];
 			wave_lds_sync();
@@ -2221,6 +2221,29 @@ __global__ __launch_bounds__(kBlock) void k_cluster_links(
 			mask[(size_t)of[p0 + lane] * kCl + i] = (uint64_t)L.row[2 * lane + 1] << 32 | L.row[2 * lane];
 		wave_lds_sync();
 	}
+}
+
+// The candidates of each of k_cluster_links' waves (measurement only): an
+// atomic on one cursor per batch doubled the search of a room of 32,768
+// patches with 215 M of them (22 -> 44 ms).
+__global__ __launch_bounds__(kBlock) void k_cluster_wave_candidates(const uint64_t* __restrict__ first,
+                                                                    const uint32_t* __restrict__ of, uint32_t split,
+                                                                    const uint64_t* __restrict__ mask,
+                                                                    uint32_t* __restrict__ count)
+{
+	constexpr uint32_t per = kCl / (kBlock / 64);
+	const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const uint32_t a = (blockIdx.x / per) >> split, part = (blockIdx.x / per) & ((1u << split) - 1u);
+	const uint32_t i = blockIdx.x % per * (kBlock / 64) + wave;
+	const uint64_t begin = first[a], partners = first[a + 1] - begin;
+	const uint64_t end = begin + (partners * (part + 1) >> split);
+	uint32_t n = 0;
+	for (uint64_t p = begin + (partners * part >> split) + lane; p < end; p += 64)
+		n += (uint32_t)__popcll(mask[(size_t)of[p] * kCl + i]);
+	for (int o = 32; o > 0; o >>= 1)
+		n += (uint32_t)__shfl_xor((int)n, o);
+	if (lane == 0)
+		count[blockIdx.x * (kBlock / 64) + wave] = n;
 }
 
 // One wave per cluster pair: its links per patch of both clusters.
@@ -4142,16 +4165,6 @@ uint64_t DeviceScene::links_by_clusters(uint32_t** colx, size_t* cap)
 		k_cluster_masks<<<gridn_waves(npairs), kBlock, 0, s>>>(W, quarters.p, mask.p, ncand.p);
 		HIPCHECK(hipGetLastError());
 		Scratch<uint64_t> at(spare_, npairs + 1);
-		Scratch<unsigned long long> cursor(spare_, 1);
-		uint2* cand = nullptr;
-		uint8_t* linked = nullptr;
-		if (count_queries) { // the candidates are kept for reference_counts_links
-			HIPCHECK(hipMemsetAsync(ncand.p + npairs, 0, 4, s));
-			scan_u32_to_u64(ncand.p, npairs + 1, at.p, &ncand_, s);
-			d_cand_ = cand = dalloc<uint2>(ncand_);
-			d_clinked_ = linked = dalloc<uint8_t>(ncand_);
-			HIPCHECK(hipMemsetAsync(cursor.p, 0, 8, s));
-		}
 		Scratch<uint32_t> flag(spare_, npairs + 1);
 		k_cluster_flags<<<grid_for(npairs + 1), kBlock, 0, s>>>(ncand.p, npairs, flag.p);
 		HIPCHECK(hipGetLastError());
@@ -4164,8 +4177,21 @@ uint64_t DeviceScene::links_by_clusters(uint32_t** colx, size_t* cap)
 			uint32_t split = 0;
 			while (split < kLinkSplitMax && ((uint64_t)Npad << split) < kLinkWaves)
 				++split;
-			k_cluster_links<<<nc * (kCl / (kBlock / 64)) << split, kBlock, 0, s>>>(
-			    V, F, first2.p, of.p, split, mask.p, cursor.p, cand, linked);
+			const uint32_t blocks = nc * (kCl / (kBlock / 64)) << split;
+			const uint64_t nwaves = (uint64_t)blocks * (kBlock / 64);
+			Scratch<uint32_t> wcount(spare_, count_queries ? nwaves + 1 : 0);
+			Scratch<uint64_t> woff(spare_, count_queries ? nwaves + 1 : 0);
+			uint2* cand = nullptr;
+			uint8_t* linked = nullptr;
+			if (count_queries) { // the candidates are kept for reference_counts_links
+				k_cluster_wave_candidates<<<blocks, kBlock, 0, s>>>(first2.p, of.p, split, mask.p, wcount.p);
+				HIPCHECK(hipGetLastError());
+				HIPCHECK(hipMemsetAsync(wcount.p + nwaves, 0, 4, s));
+				scan_u32_to_u64(wcount.p, nwaves + 1, woff.p, &ncand_, s);
+				d_cand_ = cand = dalloc<uint2>(ncand_);
+				d_clinked_ = linked = dalloc<uint8_t>(ncand_);
+			}
+			k_cluster_links<<<blocks, kBlock, 0, s>>>(V, F, first2.p, of.p, split, mask.p, woff.p, cand, linked);
 			HIPCHECK(hipGetLastError());
 			k_cluster_degrees<<<gridn_waves(nfull), kBlock, 0, s>>>(F, of.p, mask.p, deg.p);
 			HIPCHECK(hipGetLastError());

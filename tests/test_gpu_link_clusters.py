@@ -76,3 +76,25 @@ def test_automatic_choice_and_waves_per_patch(lib, n):
         assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
         assert np.array_equal(x.view(np.uint32), z.view(np.uint32))
     assert n == 2 or len(a[1]) > 1000
+
+
+@pytest.mark.parametrize("n", [1500, 9000, 40_000])
+def test_kept_candidates_are_the_all_pairs_ones(lib, n):
+    """With counting on, the clusters' candidates (16, 4 and 1 waves to a
+    patch) are those of all pairs: as many, and the canonical walk of each
+    visits as much in sum and finds the links that were kept."""
+    rng = np.random.default_rng(n)
+    pos, nrm = patches("far", n, rng)
+    tris = (pos[rng.integers(0, n, 400), None] + rng.uniform(-4, 4, (400, 3, 3))).astype(np.float32).reshape(-1, 9)
+    dev = Device(lib, tris)
+    out = []
+    for mode in (1, 2):
+        _lib.check(lib.lgx_SetCounting(dev.h, 1), lib)
+        found = len(links(lib, dev, pos, nrm, mode)[1])
+        _lib.check(lib.lgx_SetCounting(dev.h, 0), lib)
+        c = (C.c_uint64 * 5)()
+        _lib.check(lib.lgx_ReferenceCountsLinks(dev.h, P(tris), len(tris), c), lib)
+        assert c[3] == 0 and c[4] == found and c[2] > found > 50
+        out.append(list(c))
+    dev.close()
+    assert out[0] == out[1]
