@@ -215,6 +215,11 @@ LTRAPI int lgx_RadLinks(lgx_Device* dev, const float* pos3, const float* nrm3, s
  * loop does (at most 524,288 patches), mode 2 clusters.  Every mode gives the
  * same links. */
 LTRAPI int lgx_SetLinkSearch(lgx_Device* dev, int mode);
+/* No counterpart in the reference (tests). Most pairs of clusters that the
+ * search of the next lgx_RadLinks holds at a time (0, the default: what a
+ * launch and a quarter of the free memory take); with more it goes through
+ * them in runs, twice each, and finds the same links. */
+LTRAPI int lgx_SetLinkRunPairs(lgx_Device* dev, size_t pairs);
 LTRAPI int lgx_RadReadLinks(lgx_Device* dev, uint32_t* rowmap, uint32_t* other, float* factor);
 /* bounce_count rounds of Int_RDBounce (lighter.cpp:767-797) from emitted
  * light E; total3 receives the accumulated light per patch. */

@@ -78,6 +78,7 @@ LGX_SIGNATURES = {
     "lgx_DirectLightGrad": (C.c_int, [vp, C.POINTER(C.c_double), C.POINTER(C.c_double)]),
     "lgx_SetCounting": (C.c_int, [vp, C.c_int]),
     "lgx_SetLinkSearch": (C.c_int, [vp, C.c_int]),
+    "lgx_SetLinkRunPairs": (C.c_int, [vp, C.c_size_t]),
     "lgx_PrepareTimes": (C.c_int, [vp, C.POINTER(C.c_double)]),
     "lgx_SplitTreeCompare": (C.c_int, [C.POINTER(C.c_float), C.c_size_t, C.POINTER(C.c_double)]),
     "lgx_ReadCounters": (C.c_int, [vp, C.POINTER(C.c_uint64)]),

@@ -833,6 +833,12 @@ int lgx_SetLinkSearch(lgx_Device* d, int mode)
 	});
 }
 
+int lgx_SetLinkRunPairs(lgx_Device* d, size_t pairs)
+{
+	d->dev.links_run_pairs = pairs ? pairs : ~0ull;
+	return 1;
+}
+
 int lgx_SetCounting(lgx_Device* d, int on)
 {
 	d->dev.count_queries = on != 0;

@@ -214,6 +214,7 @@ public:
 	void rad_set_patches(const float* pos, const float* nrm, size_t n);
 	size_t rad_links();
 	int links_mode = 0;
+	uint64_t links_run_pairs = ~0ull; // pairs of clusters per run, at most (tests; the search has its own limit)
 	size_t rad_num_links() const { return nlinks_; }
 	// Reference link list: rowmap {offset,count} per patch, other, factor.
 	void rad_get_links(uint32_t* rowmap, uint32_t* other, float* factor) const;

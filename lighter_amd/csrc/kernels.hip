@@ -2000,19 +2000,19 @@ __device__ __forceinline__ bool may_link(const ClBox& A, const ClBox& B)
 // One wave per cluster a: its partners b >= a, super-clusters first, then
 // clusters, then the 16 pairs of quarters (four partners at a time).  Pass 0
 // counts, pass 1 writes the pair and the quarters that may link (bit 4 qa +
-// qb).
+// qb) of the clusters from a0 to a1 - 1, whose first is the pair base.
 template <bool WRITE>
 __global__ __launch_bounds__(kBlock) void k_cluster_pairs(const ClBox* __restrict__ box, const ClBox* __restrict__ quart,
                                                           uint32_t nc, const ClBox* __restrict__ sup, uint32_t ns,
-                                                          uint32_t* __restrict__ count,
-                                                          const uint64_t* __restrict__ offs, uint2* __restrict__ out,
-                                                          uint16_t* __restrict__ quarters)
+                                                          uint32_t a0, uint32_t a1, uint32_t* __restrict__ count,
+                                                          const uint64_t* __restrict__ offs, uint64_t base,
+                                                          uint2* __restrict__ out, uint16_t* __restrict__ quarters)
 {
-	const uint32_t a = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-	if (a >= nc)
+	const uint32_t a = a0 + blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+	if (a >= a1)
 		return;
 	const ClBox A = box[a], Aq = quart[4 * (size_t)a + ((lane >> 2) & 3)];
-	uint64_t at = WRITE ? offs[a] : 0;
+	uint64_t at = WRITE ? offs[a] - base : 0;
 	for (uint32_t s0 = a / kCl; s0 < ns; s0 += 64) {
 		uint64_t m = __ballot(s0 + lane < ns && may_link(A, sup[min(s0 + lane, ns - 1)]));
 		while (m) {
@@ -2094,7 +2094,8 @@ __global__ __launch_bounds__(kBlock) void k_cluster_masks(PairWork W, const uint
 }
 
 // The pairs that hold candidates, in order: their places before compaction
-// (of[], where their masks are) and the first of each cluster.
+// (of[], where their masks are) and the first of each cluster (first[p] -
+// base before).
 __global__ void k_cluster_flags(const uint32_t* __restrict__ ncand, uint64_t n, uint32_t* __restrict__ flag)
 {
 	const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2103,7 +2104,7 @@ __global__ void k_cluster_flags(const uint32_t* __restrict__ ncand, uint64_t n, 
 }
 
 __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, uint32_t nc,
-                                  const uint64_t* __restrict__ first, const uint2* __restrict__ pairs,
+                                  const uint64_t* __restrict__ first, uint64_t base, const uint2* __restrict__ pairs,
                                   uint2* __restrict__ pairs2, uint32_t* __restrict__ of, uint64_t* __restrict__ first2)
 {
 	const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2112,7 +2113,7 @@ __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, u
 		of[at[p]] = (uint32_t)p;
 	}
 	if (p <= nc)
-		first2[p] = at[first[p]];
+		first2[p] = at[first[p] - base];
 }
 
 // The occlusion tests, one wave per patch i of a cluster: its candidates in
@@ -2134,6 +2135,7 @@ __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, u
 // (whole searches: a terrain of 3,001 patches 1.27 -> 0.70 ms, of 12,001 3.77
 // -> 2.60, a room of 6,001 1.43 -> 1.10; up to twice as many gained a terrain
 // of 32,768 6.24 -> 5.72 and lost a city of 32,768 2.05 -> 2.26).
+// a0: the cluster that first[0] is of.
 // mask: the candidates' bits in, the links' out.  cand, linked (optional): the
 // candidates and whether each linked, a wave's from its candoff on.
 // The walk is one for the wave (wave_occluded).  Against a walk per lane: a room's
@@ -2145,7 +2147,7 @@ struct LinkWave {
 	uint16_t queue[128];
 };
 __global__ __launch_bounds__(kBlock) void k_cluster_links(
-    View V, PairWork W, const uint64_t* __restrict__ first, const uint32_t* __restrict__ of,
+    View V, PairWork W, uint32_t a0, const uint64_t* __restrict__ first, const uint32_t* __restrict__ of,
     uint32_t split, uint64_t* __restrict__ mask, const uint64_t* __restrict__ candoff, uint2* __restrict__ cand,
     uint8_t* __restrict__ linked)
 {
@@ -2155,7 +2157,7 @@ __global__ __launch_bounds__(kBlock) void k_cluster_links(
 	const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 	const uint32_t a = (blockIdx.x / per) >> split, part = (blockIdx.x / per) & ((1u << split) - 1u);
 	const uint32_t i = blockIdx.x % per * (kBlock / 64) + wave;
-	const float4 A = W.sp[(size_t)a * kCl + i];
+	const float4 A = W.sp[(size_t)(a0 + a) * kCl + i];
 	const uint32_t ia = __float_as_uint(A.w);
 	if (ia == kNoPatch)
 		return; // the whole wave; no block barrier below
@@ -4093,6 +4095,12 @@ void* DeviceScene::link_candidates_all(uint64_t& ncand, uint64_t* coff)
 	return cand;
 }
 
+// Most pairs of clusters and clusters of one run of the search: launches of a
+// wave for each pair and of 16 blocks for each cluster stay below 2^32
+// threads.
+constexpr uint64_t kLinkRunPairs = (1ull << 26) - 4096;
+constexpr uint32_t kLinkRunClusters = 1u << 19;
+
 // The links over clusters of patches: degrees, CSR offsets and columns (in
 // any order within a row).  Returns the entries; colx: the columns.
 uint64_t DeviceScene::links_by_clusters(uint32_t** colx, size_t* cap)
@@ -4143,67 +4151,136 @@ uint64_t DeviceScene::links_by_clusters(uint32_t** colx, size_t* cap)
 	k_cluster_boxes<<<gridn_waves(nc), kBlock, 0, s>>>(sp.p, sn.p, nc, box.p, quart.p);
 	k_super_boxes<<<gridn_waves(ns), kBlock, 0, s>>>(box.p, nc, ns, sup.p);
 	HIPCHECK(hipMemsetAsync(count.p + nc, 0, 4, s));
-	k_cluster_pairs<false><<<gridn_waves(nc), kBlock, 0, s>>>(box.p, quart.p, nc, sup.p, ns, count.p, nullptr, nullptr, nullptr);
+	k_cluster_pairs<false><<<gridn_waves(nc), kBlock, 0, s>>>(box.p, quart.p, nc, sup.p, ns, 0, nc, count.p, nullptr, 0,
+	                                                          nullptr, nullptr);
 	HIPCHECK(hipGetLastError());
 	uint64_t npairs = 0;
 	scan_u32_to_u64(count.p, (uint64_t)nc + 1, coff.p, &npairs, s);
-	if (npairs >= (1ull << 32))
-		throw std::runtime_error("radiosity: more than 2^32 cluster pairs within linking distance");
-	Scratch<uint2> pairs(spare_, npairs);
-	Scratch<uint16_t> quarters(spare_, npairs);
-	k_cluster_pairs<true><<<gridn_waves(nc), kBlock, 0, s>>>(box.p, quart.p, nc, sup.p, ns, nullptr, coff.p, pairs.p, quarters.p);
-	HIPCHECK(hipGetLastError());
-	const PairWork W{sp.p, sn.p, pairs.p, (uint32_t)npairs};
-	Scratch<uint64_t> mask(spare_, npairs * kCl);
-	Scratch<uint32_t> ncand(spare_, npairs + 1), of(spare_, npairs), deg(spare_, (uint64_t)N + 1);
-	Scratch<uint2> pairs2(spare_, npairs);
-	Scratch<uint64_t> first2(spare_, (uint64_t)nc + 1);
+	// The pairs of clusters in runs of consecutive first clusters, as many as
+	// a launch's 2^32 threads and a quarter of the free memory take (some 550
+	// bytes each): one run but for the largest scenes.  With several, each is
+	// gone through twice, for the degrees and for the columns.
+	struct Run {
+		uint32_t a0, a1;
+		uint64_t base, n; // first pair, pairs
+	};
+	std::vector<Run> runs;
+	uint64_t limit = std::min(links_run_pairs, kLinkRunPairs);
+	if (npairs > (1u << 22)) {
+		size_t free_bytes = 0, total_bytes = 0;
+		HIPCHECK(hipMemGetInfo(&free_bytes, &total_bytes));
+		limit = std::min<uint64_t>(limit, std::max<uint64_t>(free_bytes / 4 / 550, 1u << 20));
+	}
+	if (npairs <= limit && nc <= kLinkRunClusters) {
+		runs.push_back(Run{0, nc, 0, npairs});
+	} else {
+		std::vector<uint64_t> off((size_t)nc + 1);
+		HIPCHECK(hipMemcpyAsync(off.data(), coff.p, 8 * off.size(), hipMemcpyDeviceToHost, s));
+		HIPCHECK(hipStreamSynchronize(s));
+		for (uint32_t a = 0; a < nc;) {
+			uint32_t e = a + 1; // a cluster has fewer than 2^26 partners
+			while (e < nc && off[e + 1] - off[a] <= limit && e - a < kLinkRunClusters)
+				++e;
+			runs.push_back(Run{a, e, off[a], off[e] - off[a]});
+			a = e;
+		}
+	}
+	uint64_t most = 0;
+	uint32_t most_clusters = 0;
+	for (const Run& r : runs) {
+		most = std::max(most, r.n);
+		most_clusters = std::max(most_clusters, r.a1 - r.a0);
+	}
+	Scratch<uint2> pairs(spare_, most), pairs2(spare_, most);
+	Scratch<uint16_t> quarters(spare_, most);
+	Scratch<uint64_t> mask(spare_, most * kCl);
+	Scratch<uint32_t> ncand(spare_, most + 1), of(spare_, most), deg(spare_, (uint64_t)N + 1);
+	Scratch<uint64_t> first2(spare_, (uint64_t)most_clusters + 1);
 	HIPCHECK(hipMemsetAsync(deg.p, 0, 4 * ((size_t)N + 1), s));
-	uint64_t nnz = 0, nfull = 0;
-	PairWork F{sp.p, sn.p, pairs2.p, 0}; // the pairs that hold candidates
-	if (npairs) {
-		k_cluster_masks<<<gridn_waves(npairs), kBlock, 0, s>>>(W, quarters.p, mask.p, ncand.p);
+	uint32_t split = 0;
+	while (split < kLinkSplitMax && ((uint64_t)Npad << split) < kLinkWaves)
+		++split;
+	std::vector<uint64_t> run_cand(runs.size(), 0); // candidates of the runs before (counting)
+	// The pairs of run q that hold candidates, their masks the links'.  With
+	// count, its number of candidates joins ncand_; with keep, they are
+	// written to d_cand_ and d_clinked_, which a single run allocates.
+	auto search = [&](size_t q, bool count, bool keep) {
+		const Run& r = runs[q];
+		PairWork F{sp.p, sn.p, pairs2.p, 0};
+		if (!r.n)
+			return F;
+		k_cluster_pairs<true><<<gridn_waves(r.a1 - r.a0), kBlock, 0, s>>>(box.p, quart.p, nc, sup.p, ns, r.a0, r.a1,
+		                                                                  nullptr, coff.p, r.base, pairs.p, quarters.p);
 		HIPCHECK(hipGetLastError());
-		Scratch<uint64_t> at(spare_, npairs + 1);
-		Scratch<uint32_t> flag(spare_, npairs + 1);
-		k_cluster_flags<<<grid_for(npairs + 1), kBlock, 0, s>>>(ncand.p, npairs, flag.p);
+		const PairWork W{sp.p, sn.p, pairs.p, (uint32_t)r.n};
+		k_cluster_masks<<<gridn_waves(r.n), kBlock, 0, s>>>(W, quarters.p, mask.p, ncand.p);
 		HIPCHECK(hipGetLastError());
-		scan_u32_to_u64(flag.p, npairs + 1, at.p, &nfull, s);
+		Scratch<uint64_t> at(spare_, r.n + 1);
+		Scratch<uint32_t> flag(spare_, r.n + 1);
+		k_cluster_flags<<<grid_for(r.n + 1), kBlock, 0, s>>>(ncand.p, r.n, flag.p);
+		HIPCHECK(hipGetLastError());
+		uint64_t nfull = 0;
+		scan_u32_to_u64(flag.p, r.n + 1, at.p, &nfull, s);
 		F.npairs = (uint32_t)nfull;
-		k_cluster_compact<<<grid_for(std::max<uint64_t>(npairs, (uint64_t)nc + 1)), kBlock, 0, s>>>(
-		    npairs, at.p, nc, coff.p, pairs.p, pairs2.p, of.p, first2.p);
+		const uint32_t ncl = r.a1 - r.a0;
+		k_cluster_compact<<<grid_for(std::max<uint64_t>(r.n, (uint64_t)ncl + 1)), kBlock, 0, s>>>(
+		    r.n, at.p, ncl, coff.p + r.a0, r.base, pairs.p, pairs2.p, of.p, first2.p);
 		HIPCHECK(hipGetLastError());
 		if (nfull) {
-			uint32_t split = 0;
-			while (split < kLinkSplitMax && ((uint64_t)Npad << split) < kLinkWaves)
-				++split;
-			const uint32_t blocks = nc * (kCl / (kBlock / 64)) << split;
+			const uint32_t blocks = ncl * (kCl / (kBlock / 64)) << split;
 			const uint64_t nwaves = (uint64_t)blocks * (kBlock / 64);
-			Scratch<uint32_t> wcount(spare_, count_queries ? nwaves + 1 : 0);
-			Scratch<uint64_t> woff(spare_, count_queries ? nwaves + 1 : 0);
-			uint2* cand = nullptr;
-			uint8_t* linked = nullptr;
-			if (count_queries) { // the candidates are kept for reference_counts_links
+			Scratch<uint32_t> wcount(spare_, count || keep ? nwaves + 1 : 0);
+			Scratch<uint64_t> woff(spare_, count || keep ? nwaves + 1 : 0);
+			if (count || keep) {
+				uint64_t n = 0;
 				k_cluster_wave_candidates<<<blocks, kBlock, 0, s>>>(first2.p, of.p, split, mask.p, wcount.p);
 				HIPCHECK(hipGetLastError());
 				HIPCHECK(hipMemsetAsync(wcount.p + nwaves, 0, 4, s));
-				scan_u32_to_u64(wcount.p, nwaves + 1, woff.p, &ncand_, s);
-				d_cand_ = cand = dalloc<uint2>(ncand_);
-				d_clinked_ = linked = dalloc<uint8_t>(ncand_);
+				scan_u32_to_u64(wcount.p, nwaves + 1, woff.p, &n, s);
+				if (count) {
+					run_cand[q] = ncand_;
+					ncand_ += n;
+				}
+				if (keep && count) {
+					d_cand_ = dalloc<uint2>(ncand_);
+					d_clinked_ = dalloc<uint8_t>(ncand_);
+				}
 			}
-			k_cluster_links<<<blocks, kBlock, 0, s>>>(V, F, first2.p, of.p, split, mask.p, woff.p, cand, linked);
+			k_cluster_links<<<blocks, kBlock, 0, s>>>(V, F, r.a0, first2.p, of.p, split, mask.p, woff.p,
+			                                          keep ? (uint2*)d_cand_ + run_cand[q] : nullptr,
+			                                          keep ? (uint8_t*)d_clinked_ + run_cand[q] : nullptr);
 			HIPCHECK(hipGetLastError());
-			k_cluster_degrees<<<gridn_waves(nfull), kBlock, 0, s>>>(F, of.p, mask.p, deg.p);
+			HIPCHECK(hipStreamSynchronize(s)); // before at .. woff go
+		}
+		return F;
+	};
+	const bool one = runs.size() == 1;
+	PairWork F{sp.p, sn.p, pairs2.p, 0};
+	for (size_t q = 0; q < runs.size(); ++q) {
+		F = search(q, count_queries, count_queries && one);
+		if (F.npairs) {
+			k_cluster_degrees<<<gridn_waves(F.npairs), kBlock, 0, s>>>(F, of.p, mask.p, deg.p);
 			HIPCHECK(hipGetLastError());
 		}
-		HIPCHECK(hipStreamSynchronize(s)); // before at .. flag go
 	}
+	uint64_t nnz = 0;
 	scan_u32_to_u64(deg.p, (uint64_t)N + 1, rad.rowptr64, &nnz, s);
 	*colx = (uint32_t*)spare_.take(4 * nnz, cap);
-	if (nnz) {
+	const bool keep = count_queries && !one && ncand_;
+	if (keep) {
+		d_cand_ = dalloc<uint2>(ncand_);
+		d_clinked_ = dalloc<uint8_t>(ncand_);
+	}
+	if (nnz || keep) {
 		HIPCHECK(hipMemsetAsync(deg.p, 0, 4 * ((size_t)N + 1), s)); // the rows' cursors
-		k_cluster_fill<<<gridn_waves(nfull), kBlock, 0, s>>>(F, of.p, mask.p, rad.rowptr64, deg.p, *colx);
-		HIPCHECK(hipGetLastError());
+		for (size_t q = 0; q < runs.size(); ++q) {
+			if (!one)
+				F = search(q, false, keep);
+			if (F.npairs && nnz) {
+				k_cluster_fill<<<gridn_waves(F.npairs), kBlock, 0, s>>>(F, of.p, mask.p, rad.rowptr64, deg.p, *colx);
+				HIPCHECK(hipGetLastError());
+			}
+		}
 	}
 	HIPCHECK(hipStreamSynchronize(s)); // before the arrays here go
 	return nnz;

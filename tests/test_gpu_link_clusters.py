@@ -98,3 +98,29 @@ def test_kept_candidates_are_the_all_pairs_ones(lib, n):
         out.append(list(c))
     dev.close()
     assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("run", [1, 37, 500])
+def test_runs_of_cluster_pairs(lib, run):
+    """A search that takes its pairs of clusters in many runs (one first
+    cluster each, a few, some more) against one run: links, factors and
+    the candidates kept with counting on."""
+    n = 9000
+    rng = np.random.default_rng(run)
+    pos, nrm = patches("far", n, rng)
+    tris = (pos[rng.integers(0, n, 400), None] + rng.uniform(-4, 4, (400, 3, 3))).astype(np.float32).reshape(-1, 9)
+    dev = Device(lib, tris)
+    out = []
+    for pairs in (0, run):
+        _lib.check(lib.lgx_SetLinkRunPairs(dev.h, pairs), lib)
+        got = links(lib, dev, pos, nrm, 2)
+        _lib.check(lib.lgx_SetCounting(dev.h, 1), lib)
+        links(lib, dev, pos, nrm, 2)
+        _lib.check(lib.lgx_SetCounting(dev.h, 0), lib)
+        c = (C.c_uint64 * 5)()
+        _lib.check(lib.lgx_ReferenceCountsLinks(dev.h, P(tris), len(tris), c), lib)
+        out.append((*got, np.array(list(c), np.uint64).view(np.uint32)))
+    dev.close()
+    assert len(out[0][1]) > 1000
+    for x, y in zip(*out):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
