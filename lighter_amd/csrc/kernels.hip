@@ -1569,18 +1569,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 	ao_blend(s, ao, P, lm, fac_out);
 }
 
-// The same for at most 32 rays: T = 64 / n texels per wave, lane q n + i the
+// The same for at most 32 rays: T <= 64 / n texels per wave, lane q n + i the
 // i-th ray of its q-th texel.  Bound by the walks' node fetches as k_ao is;
 // a wave per texel left 47 lanes idle at 17 rays (a city's 700,001 texels
 // 1.97 ms; packed 0.90).  Above 32 rays no second texel fits.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_ao_packed(
     View V, const float* __restrict__ pos, const float* __restrict__ nrm, const float* __restrict__ randoff,
-    const float2* __restrict__ side, AOParams P, uint32_t s0, uint32_t S, float* __restrict__ lm, int depth,
-    float* __restrict__ fac_out)
+    const float2* __restrict__ side, AOParams P, uint32_t T, uint32_t s0, uint32_t S, float* __restrict__ lm,
+    int depth, float* __restrict__ fac_out)
 {
 	extern __shared__ __align__(16) unsigned char lds_stack[];
 	LdsStack st = lds_stack_of_lane(lds_stack, depth);
-	const uint32_t lane = threadIdx.x & 63, n = (uint32_t)P.n, T = 64 / n;
+	const uint32_t lane = threadIdx.x & 63, n = (uint32_t)P.n;
 	const uint32_t q = lane / n, i = lane - q * n;
 	const uint32_t s = s0 + (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * T + q;
 	const bool in = q < T && s < S;
@@ -3916,14 +3916,23 @@ void DeviceScene::ambient_occlusion(const float* randoff, int num_samples, float
 	// one launch, or, when the caller follows progress, chunks of texels
 	// with the caller asked between them whether to go on
 	const size_t chunk = between ? kAOChunk : nsamples_;
+	const size_t resident = (size_t)persistent_blocks() * (kBlock / 64);
 	EventTimer tm(s);
 	for (size_t b = 0; b < nsamples_; b += chunk) {
 		const size_t e = std::min(nsamples_, b + chunk);
 		const unsigned ao_grid = (unsigned)((e - b + kBlock / 64 - 1) / (kBlock / 64)); // a wave per texel
-		if (!count_queries && num_samples <= 32) {
-			const size_t per = (size_t)(kBlock / 64) * (64 / num_samples); // texels per block
+		// Texels per wave: three for each texel per wave that fits the chip
+		// (6,144), since waves that would fit find the chip idle.  One ray
+		// of 2,001 texels in a city: 64 to a wave 56 us, one 40; 17 rays of
+		// 6,001 texels in a terrain: three 69 us, one 80; over 301 .. 300,001
+		// texels and 1 .. 32 rays twice and four times as many were 0.3 and
+		// 1 % slower in the mean.
+		const size_t T = std::min<size_t>(64 / num_samples, (3 * (e - b) + resident - 1) / resident);
+		if (!count_queries && T > 1) {
+			const size_t per = (size_t)(kBlock / 64) * T; // texels per block
 			k_ao_packed<<<(unsigned)((e - b + per - 1) / per), kBlock, march_lds_bytes(), s>>>(
-			    V, d_pos_, d_nrm_, d_ro, d_side, P, (uint32_t)b, (uint32_t)e, d_lm_, march_stack_depth(), fac_out);
+			    V, d_pos_, d_nrm_, d_ro, d_side, P, (uint32_t)T, (uint32_t)b, (uint32_t)e, d_lm_, march_stack_depth(),
+			    fac_out);
 		} else if (count_queries)
 			k_ao<true><<<ao_grid, kBlock, march_lds_bytes(), s>>>(V, d_pos_, d_nrm_, d_ro, d_side, P, (uint32_t)b,
 			                                                      (uint32_t)e, d_lm_, d_counters_,

@@ -1,6 +1,6 @@
 """Ambient occlusion with several texels to a wave (at most 32 rays each)
 against a wave per texel, which a device that counts its queries takes for
-every ray count: the same rays and the same order of their sum, so the colours
+every ray count (from 2,049 texels on, the more texels the more to a wave): the same rays and the same order of their sum, so the colours
 agree bit for bit (Job_AORender_Inner, lighter.cpp:799-841)."""
 
 import ctypes as C
@@ -20,7 +20,7 @@ def _soup(rng, n):
 
 
 @pytest.mark.parametrize("rays", [1, 2, 3, 17, 21, 22, 31, 32, 33, 64, 65])
-@pytest.mark.parametrize("texels", [1, 5, 1001])
+@pytest.mark.parametrize("texels", [1, 5, 1001, 7001, 140_001])
 def test_packed_texels_match_wave_per_texel(lib, rays, texels):
     rng = np.random.default_rng(100 * rays + texels)
     dev = Device(lib, _soup(rng, 300))
