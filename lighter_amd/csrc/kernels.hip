@@ -890,7 +890,9 @@ struct DirectSrc { // the marches of the direct light: work items, neighbours in
 };
 
 struct QuerySrc { // the marches of lgx_QueryShadow, in the caller's order: lanes of a wave far apart
-	// 100,003 in a terrain: 1.48 ms with waves, 1.63 on lanes; 200,003: 2.8 and 2.2
+	// whole calls with waves and on lanes, ms: 100,003 scattered in a city 1.21
+	// and 2.01, in a terrain 1.79 and 1.91; 131,001: 1.51 and 1.94, 2.25 and
+	// 1.86
 	static constexpr uint32_t kWaveMax = 1u << 17;
 	const float* __restrict__ from;
 	const float* __restrict__ to;
@@ -1570,9 +1572,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 }
 
 // The same for at most 32 rays: T <= 64 / n texels per wave, lane q n + i the
-// i-th ray of its q-th texel.  Bound by the walks' node fetches as k_ao is;
-// a wave per texel left 47 lanes idle at 17 rays (a city's 700,001 texels
-// 1.97 ms; packed 0.90).  Above 32 rays no second texel fits.
+// i-th ray of its q-th texel.  Bound by the walks' instruction issue as k_ao is
+// (0.28 VALU instructions per SIMD-cycle, 82 % L2 hits); a wave per texel left
+// 47 lanes idle at 17 rays (a city's 700,001 texels 1.97 ms; packed 0.90).
+// Above 32 rays no second texel fits.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_ao_packed(
     View V, const float* __restrict__ pos, const float* __restrict__ nrm, const float* __restrict__ randoff,
     const float2* __restrict__ side, AOParams P, uint32_t T, uint32_t s0, uint32_t S, float* __restrict__ lm,
@@ -2056,7 +2059,9 @@ struct PairWork {
 // One wave per cluster pair: the bit matrix of the pairs that pass
 // pair_factor (row: a patch of the first cluster) and their number.  A lane
 // keeps its patch of the second cluster; the first cluster's patches are
-// uniform.  Bound by instruction issue, about 30 a pair of patches.
+// uniform.  Bound by instruction issue, about 30 a pair of patches (0.23-0.27
+// VALU and 0.09 scalar instructions per SIMD-cycle, 11-14 % of the wave-cycles
+// waiting).
 __global__ __launch_bounds__(kBlock) void k_cluster_masks(PairWork W, const uint16_t* __restrict__ quarters,
                                                           uint64_t* __restrict__ mask, uint32_t* __restrict__ ncand)
 {
@@ -2125,8 +2130,9 @@ __global__ void k_cluster_compact(uint64_t n, const uint64_t* __restrict__ at, u
 // share one end, and the other ends go along the clusters' Morton order, so
 // their walks take much the same nodes (batches per cluster pair, some seven
 // patches of the first cluster in each, took 19.3 ms instead of 16.4 on a
-// city of 440,003 patches with 139 M candidates).  Bound by the walks' issue
-// and node fetches.  A city's whole search, kernels: 50 ms with a uniform
+// city of 440,003 patches with 139 M candidates).  Bound by the walks'
+// instruction issue (0.33 VALU and 0.14-0.15 scalar instructions per
+// SIMD-cycle; 95 % of the fetches hit the L2).  A city's whole search, kernels: 50 ms with a uniform
 // grid's candidate list (30.1 ms of pair tests, made twice; 12.6 ms of
 // occlusion tests on the list), 26 ms so (pair tests 2.4 ms); a room's 20 ->
 // 12 ms.
