@@ -782,15 +782,18 @@ class DirectLeg:
                     kernel="k_march", alg_bytes_per_launch=int(alg), kernel_ms=round(self.march_avg, 3),
                     note="reference-shaped count: the same marches on a plain binary SAH tree (16 bins, <= 4 "
                          "triangles per leaf) with one radius-2 distance query per step, node visits x 32 B + "
-                         "triangle tests x 36 B, plus 36 B of I/O per item, over the march kernel's average "
-                         "HIP-event duration; traffic: HBM bytes per launch from rocprofv3 FETCH_SIZE/WRITE_SIZE",
+                         "triangle tests x 36 B, plus 36 B of I/O per item, over the march kernels' average "
+                         "HIP-event duration (k_march and the k_march_wave that finishes its long marches; the "
+                         "product reads fewer bytes, mostly from the caches, so the rate can exceed HBM's); "
+                         "traffic: HBM bytes of both from rocprofv3 FETCH_SIZE/WRITE_SIZE",
                     reference_counts=dict(node_visits=rvis, triangle_tests=rtri, distance_queries=rq, marches=rm,
                                           factors_differing=rbad),
                     this_build=dict(node_visits=self.nodes, triangle_tests=self.ntests, box_pretests=self.npre,
                                     distance_queries=self.qsteps, bytes_per_launch=int(own),
                                     achieved_gbs=round(own / (self.march_avg / 1000.0) / 1e9, 1),
                                     note="4-wide nodes x 112 B + full triangle tests x 160 B + box pre-tests x "
-                                         "48 B + I/O on this build's own tree and query bounds"))
+                                         "48 B + I/O on this build's own tree and query bounds, as counted with "
+                                         "every march on its lane"))
 
     def cpu(self, seconds, cores_info, ao=None):
         """CPU leg: the reference's CalcInvShadowFactor on a seeded sample of
